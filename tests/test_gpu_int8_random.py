@@ -86,3 +86,27 @@ def test_int8_few_rows_k_split_is_repeatable(orc, plan):
         M_.i8mm_launch(a[:rows].contiguous(), b, bias, right_transpose=True, acc=acc)
         torch.cuda.synchronize()
         assert np.array_equal(acc.cpu().numpy().astype(np.int64), want[:rows]), rows
+
+
+@pytest.mark.parametrize("tile,ring", [(128, 64), (128, 4), (256, 0)])
+@pytest.mark.parametrize("M,K,N", [(1, 1, 1), (129, 63, 130), (130, 65, 129), (128, 127, 257), (257, 192, 143), (40, 1000, 300)])
+@pytest.mark.parametrize("rt", [True, False])
+def test_rewritten_operands_and_folded_zero_points(orc, plan, tile, ring, M, K, N, rt):
+    """K that is no whole number of stages (padded), [K, N] right operands (transposed), unsigned bytes and both zero
+    points, in each tile kernel, with the unsigned 8-bit Q31 output; row pieces at every alignment (odd K and N)."""
+    import torch
+    plan(i8_tile=tile, i8_mid_ring=ring)
+    c = S.int8_matmul(M, K, N, seed=900 + M, right_transpose=rt)
+    a, b = c["a"].view(np.uint8), c["b"].view(np.uint8)
+    dev = lambda t: torch.from_numpy(np.ascontiguousarray(t)).cuda()
+    zp = np.arange(N, dtype=np.int32) % 40
+    rq = M_.RequantDesc(clib.RQ_QDM, clib.ROUND_HALF_AWAY_FROM_ZERO, out_dtype=clib.DT_U8, multiplier=dev(c["mult"]),
+                        shift=dev(c["shift"]), zp=dev(zp))
+    acc = torch.empty((M, N), dtype=torch.int32, device="cuda")
+    out = M_.i8mm_launch(dev(a), dev(b), dev(c["bias"]), right_transpose=rt, input_zp=117, right_zp=140, rq=rq, acc=acc)
+    torch.cuda.synchronize()
+    want = (a.astype(np.int64) - 117) @ ((b.T if rt else b).astype(np.int64) - 140) + c["bias"].astype(np.int64)
+    assert np.array_equal(acc.cpu().numpy().astype(np.int64), want)
+    v = orc.mbqm(want.astype(np.int32), np.broadcast_to(c["mult"], want.shape),
+                 -np.broadcast_to(c["shift"], want.shape), orc.HALF_AWAY_FROM_ZERO).astype(np.int64)
+    assert np.array_equal(out.cpu().numpy().astype(np.int64), np.clip(v + zp, 0, 255))

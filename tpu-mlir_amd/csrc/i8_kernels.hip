@@ -5,7 +5,7 @@
 // lib/Dialect/Tpu/Interfaces/Common/MatMul.cpp:598-604), which is exact while partial sums stay below 2^24; on
 // that domain int32 accumulation is bit-identical.  Zero points are folded algebraically:
 //   sum (a - izp)(b - rzp) = sum a*b - izp * colsum_b[n] - rzp * rowsum_a[m] + K * izp * rzp
-// and uint8 operands are re-biased to int8 (x ^ 0x80, zero point - 128) while they are staged into LDS.
+// and uint8 operands are re-biased to int8 (x ^ 0x80, zero point - 128) on their way into the matrix instructions.
 #include <stdlib.h>
 
 #include "device_math.h"
@@ -20,24 +20,6 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 // ------------------------------------------------------------------------------------------------
 // small helper kernels
 // ------------------------------------------------------------------------------------------------
-// dst[N,K] = src[K,N]^T (bytes)
-__global__ void transpose_bytes_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int64_t K,
-                                       int64_t N) {
-  __shared__ uint8_t tile[64][65];
-  const int64_t n0 = (int64_t)blockIdx.x * 64, k0 = (int64_t)blockIdx.y * 64;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 256 threads: 64 x 4
-  for (int r = ty; r < 64; r += 4) {
-    int64_t k = k0 + r, n = n0 + tx;
-    tile[r][tx] = (k < K && n < N) ? src[k * N + n] : 0;
-  }
-  __syncthreads();
-  for (int r = ty; r < 64; r += 4) {
-    int64_t n = n0 + r, k = k0 + tx;
-    if (n < N && k < K)
-      dst[n * K + k] = tile[tx][r];
-  }
-}
-
 // The two layout changes MatMul::run applies to operands and outputs (lib/Support/Dnnl/MatMul.cpp:167-239).  One
 // thread per destination element; T = uint8_t (operands) or int32_t (accumulators).
 // mode 0, tensor_hw_transpose: src [NC, H, W] -> dst [NC, W, H];  mode 1, tensor_hc_transpose: src [N, C, H, W] ->
@@ -77,215 +59,158 @@ int permute_launch(const void *d_src, void *d_dst, int elem_bytes, int mode, int
   return MI_SUCCESS;
 }
 
-// dst = src ^ 0x80 per byte: an unsigned operand u becomes the signed value u - 128 the matrix cores take
-__global__ void flip_bytes_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int64_t n) {
-  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 16;
-  if (i + 16 <= n) {
-    u32x4 v = *(const u32x4 *)(src + i);
-    v[0] ^= 0x80808080u;
-    v[1] ^= 0x80808080u;
-    v[2] ^= 0x80808080u;
-    v[3] ^= 0x80808080u;
-    *(u32x4 *)(dst + i) = v;
+// ------------------------------------------------------------------------------------------------
+// Operands that the tile kernels cannot take as they lie in memory are rewritten once, both in one launch: a [K, N]
+// right operand becomes [N, K], a K that is not a whole number of K stages is padded to one, and (for the kernel that
+// cannot do it on the way to the matrix cores) unsigned bytes are re-biased to signed.  HBM / launch bound: every
+// byte is read and written once, in 16-byte pieces whatever the row alignment (a piece that would reach past its row
+// is put together from bytes).  1000 x 3000 transposed + 333 x 1000 padded: 7.4 us, both operands; the 64 x 64
+// byte-wise transpose it replaces took 10 us for the right operand alone, and the register-staged kernel that took any
+// K without padding 182 us for that product where the ring kernel below takes 14 (437 us at 333 x 1000 x 3000, now 18).
+// ------------------------------------------------------------------------------------------------
+struct I8Copy {
+  const uint8_t *src;
+  uint8_t *dst;        // [rows][Kp]
+  int64_t rows, K, Kp;
+  int64_t blocks;      // workgroups that share this operand; 0: it is used where it is
+  int transpose;       // src is [K][rows], else [rows][K]
+  uint32_t flip4;      // XORed into every dword
+  uint32_t pad4;       // what k >= K holds
+};
+
+// 16 bytes of a row of `len` bytes from position `at`: bytes past the end are `pad`
+__device__ __forceinline__ u32x4 load16_ragged(const uint8_t *row, int64_t at, int64_t len, uint32_t pad4) {
+  u32x4 v = {pad4, pad4, pad4, pad4};
+  if (at + 16 <= len) {
+    __builtin_memcpy(&v, row + at, 16);
+  } else if (at < len) {
+    uint32_t w[4] = {pad4, pad4, pad4, pad4};
+    for (int i = 0; i < 16 && at + i < len; ++i) {
+      const int sh = 8 * (i & 3);
+      w[i >> 2] = (w[i >> 2] & ~(0xffu << sh)) | ((uint32_t)row[at + i] << sh);
+    }
+    v = u32x4{w[0], w[1], w[2], w[3]};
+  }
+  return v;
+}
+
+__device__ __forceinline__ void copy_rows(const I8Copy &c, int64_t block) {
+  const uint32_t cpr = (uint32_t)(c.Kp / 16);
+  const int64_t i = block * 256 + threadIdx.x;
+  const int64_t r = c.blocks < (1 << 24) ? (int64_t)((uint32_t)i / cpr) : i / cpr;  // a 64-bit division costs more than the copy
+  if (r >= c.rows)
+    return;
+  const int64_t k = (i - r * cpr) * 16;
+  u32x4 v = load16_ragged(c.src + r * c.K, k, c.K, c.pad4 ^ c.flip4);
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    v[e] ^= c.flip4;
+  *(u32x4 *)(c.dst + r * c.Kp + k) = v;
+}
+
+// 128 k x 128 n per workgroup: a thread reads 16 bytes of each of four consecutive k rows, turns them into 16 dwords
+// of four k each (two byte permutes per dword) and leaves those in LDS, from where rows of n go out 128 bytes at a time
+__device__ __forceinline__ void copy_transposed(const I8Copy &c, int64_t block, uint32_t (*tile)[33]) {
+  const int tid = threadIdx.x;
+  const int64_t nb = (c.rows + 127) / 128;
+  const int64_t n0 = block % nb * 128, k0 = block / nb * 128;
+  {
+    const int nc = tid & 7, kq = tid >> 3;
+    const int64_t n = n0 + nc * 16, k = k0 + kq * 4;
+    u32x4 w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const uint32_t raw = c.pad4 ^ c.flip4;
+      w[u] = k + u < c.K ? load16_ragged(c.src + (k + u) * c.rows, n, c.rows, raw) : u32x4{raw, raw, raw, raw};
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const uint32_t a = __builtin_amdgcn_perm(w[1][d], w[0][d], 0x05010400u), b = __builtin_amdgcn_perm(w[3][d], w[2][d], 0x05010400u);
+      const uint32_t e = __builtin_amdgcn_perm(w[1][d], w[0][d], 0x07030602u), f = __builtin_amdgcn_perm(w[3][d], w[2][d], 0x07030602u);
+      tile[nc * 16 + 4 * d + 0][kq] = __builtin_amdgcn_perm(b, a, 0x05040100u) ^ c.flip4;
+      tile[nc * 16 + 4 * d + 1][kq] = __builtin_amdgcn_perm(b, a, 0x07060302u) ^ c.flip4;
+      tile[nc * 16 + 4 * d + 2][kq] = __builtin_amdgcn_perm(f, e, 0x05040100u) ^ c.flip4;
+      tile[nc * 16 + 4 * d + 3][kq] = __builtin_amdgcn_perm(f, e, 0x07060302u) ^ c.flip4;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < 4; ++it) {
+    const int r = it * 32 + (tid >> 3), ch = tid & 7;
+    const int64_t n = n0 + r, k = k0 + ch * 16;
+    if (n < c.rows && k < c.Kp)
+      *(u32x4 *)(c.dst + n * c.Kp + k) = u32x4{tile[r][4 * ch], tile[r][4 * ch + 1], tile[r][4 * ch + 2], tile[r][4 * ch + 3]};
+  }
+}
+
+__global__ __launch_bounds__(256) void i8_prepare_kernel(I8Copy a, I8Copy b) {
+  __shared__ uint32_t tile[128][33];
+  if ((int64_t)blockIdx.x < b.blocks) {
+    if (b.transpose)
+      copy_transposed(b, blockIdx.x, tile);
+    else
+      copy_rows(b, blockIdx.x);
   } else {
-    for (int64_t j = i; j < n; ++j)
-      dst[j] = src[j] ^ 0x80;
+    copy_rows(a, (int64_t)blockIdx.x - b.blocks);
   }
 }
 
-// sums[r] = sum_k (signed or unsigned) x[r, k]; one wave per row
-__global__ void row_sums_kernel(const uint8_t *__restrict__ x, int is_unsigned, int32_t *__restrict__ sums,
-                                int64_t rows, int64_t K) {
+// Zero points of the large-tile kernel, which takes them as an effective bias per column and a term per row: one wave
+// per row of B, then of A (both signed by now, K a multiple of 16; padding bytes are zero).  kzz = K * izp * rzp over
+// the K of the caller.  (The smaller kernels form the same sums from the fragments they multiply.)
+__device__ __forceinline__ int32_t sum_bytes(u32x4 v, int32_t s) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    s = __builtin_amdgcn_sdot4((int)v[e], 0x01010101, s, false);
+  return s;
+}
+__global__ __launch_bounds__(256) void i8_zero_terms_kernel(const uint8_t *__restrict__ A, const uint8_t *__restrict__ B,
+                                                            int64_t M, int64_t N, int64_t K, int32_t izp, int32_t rzp,
+                                                            int32_t kzz, const int32_t *__restrict__ bias,
+                                                            int32_t *__restrict__ bias_eff, int32_t *__restrict__ row_term) {
   const int lane = threadIdx.x & 63;
-  const int64_t r = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (r >= rows)
+  int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const bool is_b = r < N;
+  if (!is_b)
+    r -= N;
+  if (!is_b && (r >= M || !row_term))
     return;
+  const uint8_t *row = (is_b ? B : A) + r * K;
   int32_t s = 0;
-  for (int64_t k = lane; k < K; k += 64) {
-    uint8_t b = x[r * K + k];
-    s += is_unsigned ? (int32_t)b : (int32_t)(int8_t)b;
-  }
+  for (int64_t k = lane * 16; k < K; k += 64 * 16)
+    s = sum_bytes(*(const u32x4 *)(row + k), s);
+#pragma unroll
   for (int off = 32; off > 0; off >>= 1)
-    s += __shfl_down(s, off, 64);
-  if (lane == 0)
-    sums[r] = s;
+    s += __shfl_xor(s, off, 64);
+  if (lane == 0) {
+    if (is_b)
+      bias_eff[r] = (bias ? bias[r] : 0) - izp * s + kzz;
+    else
+      row_term[r] = -rzp * s;
+  }
 }
-
-// Zero-point folding.  With a' = a - 128*ua (uint8 operands re-biased to int8), izp' = input_zp - 128*ua and the
-// same for b:  sum_k (a - input_zp)(b - right_zp) = sum a'b' - izp' * sum_k b'[n,k] - rzp' * sum_k a'[m,k]
-// + K * izp' * rzp'.  sums_raw are over the bytes as stored; `sub` = 128*K turns them into sums of a'/b'.
-__global__ void fold_bias_kernel(const int32_t *__restrict__ bias, const int32_t *__restrict__ colsum_raw,
-                                 int32_t *__restrict__ bias_eff, int64_t N, int64_t izp, int64_t rzp, int64_t K,
-                                 int64_t sub) {
-  int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N)
-    return;
-  int64_t v = bias ? bias[n] : 0;
-  if (colsum_raw)
-    v -= izp * ((int64_t)colsum_raw[n] - sub);
-  v += K * izp * rzp;
-  bias_eff[n] = (int32_t)v;
-}
-
-__global__ void row_term_kernel(const int32_t *__restrict__ rowsum_raw, int32_t *__restrict__ row_term, int64_t M,
-                                int64_t rzp, int64_t sub) {
-  int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m < M)
-    row_term[m] = (int32_t)(-rzp * ((int64_t)rowsum_raw[m] - sub));
-}
-
-// ------------------------------------------------------------------------------------------------
-// GEMM kernel: C[M,N] = A[M,K] * B[N,K]^T, 128x128 tile per workgroup, 4 waves (2x2), each wave a 64x64
-// sub-tile as 2x2 MFMA 32x32x32 blocks.  K is consumed 64 bytes at a time through two LDS stages.
-// LDS rows are padded to 80 bytes: 16-byte chunk slots (5*row + c) mod 16 are distinct for 16 consecutive rows,
-// so the 16-byte-per-lane fragment reads are bank-conflict free.
-// ------------------------------------------------------------------------------------------------
-constexpr int BM = 128, BN = 128, BK = 64;
-constexpr int LDS_ROW = 80;
 
 struct I8Args {
   const uint8_t *A;
   const uint8_t *B;
-  const int32_t *bias;     // effective bias [N] or null
-  const int32_t *row_term; // -rzp * rowsum_a[m] or null
+  const int32_t *bias;     // [N] or null; the large kernel's holds the zero-point terms of its column
+  const int32_t *row_term; // large kernel: -rzp * rowsum_a[m] or null
   void *out;
   int32_t *acc_out;
-  int64_t M, K, N;
-  int a_flip, b_flip;  // XOR applied to each byte (0x80 for unsigned operands)
+  int64_t M, K, N;         // K as the operands are laid out, padding included
+  uint32_t a_flip4, b_flip4;  // XOR applied to each byte (0x80 for unsigned operands)
+  int32_t izp, rzp, kzz;      // zero points of the re-biased operands; K * izp * rzp
   int do_relu;
   int64_t relu_limit;
   int has_rq;
-  int q31_half_away;  // the requantization is the Q31 multiplier / right shift in [1, 31] / half away / int8 case
+  int q31_half_away;  // the requantization is the Q31 multiplier / right shift in [1, 31] / half away / 8-bit case
+  int out_u8;         // ... with unsigned bytes out
   RequantParams rq;
   // few-row kernel only: K shared by 2^split_shift workgroups per 32-column block (0: none of the below is touched)
   int split_shift;
   int32_t *part;       // [workgroup][16 registers][64 lanes]
   unsigned *counters;  // [block], zero between launches
 };
-
-__device__ __forceinline__ u32x4 load_chunk(const uint8_t *base, int64_t row, int64_t rows, int64_t k, int64_t K,
-                                            uint32_t flip4, bool vec_ok) {
-  u32x4 v = {0, 0, 0, 0};
-  if (row < rows && k < K) {
-    const uint8_t *p = base + row * K + k;
-    if (vec_ok && k + 16 <= K) {
-      v = *(const u32x4 *)p;
-      v[0] ^= flip4;
-      v[1] ^= flip4;
-      v[2] ^= flip4;
-      v[3] ^= flip4;
-    } else {
-      uint8_t tmp[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        tmp[i] = (k + i < K) ? (uint8_t)(p[i] ^ (uint8_t)flip4) : (uint8_t)0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[i] = (uint32_t)tmp[4 * i] | ((uint32_t)tmp[4 * i + 1] << 8) | ((uint32_t)tmp[4 * i + 2] << 16) |
-               ((uint32_t)tmp[4 * i + 3] << 24);
-    }
-  }
-  return v;
-}
-
-__global__ __launch_bounds__(256) void i8_gemm_kernel(I8Args a) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds_a[2][BM * LDS_ROW];
-  __shared__ __attribute__((aligned(16))) uint8_t lds_b[2][BN * LDS_ROW];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int64_t m_base = (int64_t)blockIdx.y * BM, n_base = (int64_t)blockIdx.x * BN;
-  const bool vec_ok = (a.K % 16) == 0;
-  const uint32_t aflip = (uint32_t)a.a_flip * 0x01010101u, bflip = (uint32_t)a.b_flip * 0x01010101u;
-
-  // staging: 128 rows x 4 chunks of 16 B per operand tile = 512 chunks, two per thread
-  const int c_row0 = tid >> 2, c_col = tid & 3;  // rows c_row0 and c_row0 + 64
-  u32x4 ra[2], rb[2];
-  auto gload = [&](int64_t k0) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      ra[h] = load_chunk(a.A, m_base + c_row0 + 64 * h, a.M, k0 + 16 * c_col, a.K, aflip, vec_ok);
-      rb[h] = load_chunk(a.B, n_base + c_row0 + 64 * h, a.N, k0 + 16 * c_col, a.K, bflip, vec_ok);
-    }
-  };
-  auto lstore = [&](int stage) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      *(u32x4 *)&lds_a[stage][(c_row0 + 64 * h) * LDS_ROW + 16 * c_col] = ra[h];
-      *(u32x4 *)&lds_b[stage][(c_row0 + 64 * h) * LDS_ROW + 16 * c_col] = rb[h];
-    }
-  };
-
-  i32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        acc[i][j][r] = 0;
-
-  const int64_t k_iters = (a.K + BK - 1) / BK;
-  gload(0);
-  lstore(0);
-  __syncthreads();
-  const int frow = lane & 31, fk = (lane >> 5) * 16;
-  for (int64_t it = 0; it < k_iters; ++it) {
-    const int stage = (int)(it & 1);
-    if (it + 1 < k_iters)
-      gload((it + 1) * BK);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      i32x4 fa[2], fb[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        fa[i] = *(const i32x4 *)&lds_a[stage][(wm * 64 + i * 32 + frow) * LDS_ROW + ks * 32 + fk];
-        fb[i] = *(const i32x4 *)&lds_b[stage][(wn * 64 + i * 32 + frow) * LDS_ROW + ks * 32 + fk];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
-    }
-    if (it + 1 < k_iters) {
-      lstore(stage ^ 1);
-      __syncthreads();
-    }
-  }
-
-  // epilogue: 32x32 block layout -- register r of lane l is row 8*(r/4) + 4*(l/32) + (r%4), column l%32.  The loops
-  // carry no early exits so that they unroll completely and the accumulators stay in registers.
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int64_t n = n_base + wn * 64 + j * 32 + (lane & 31);
-    const bool n_ok = n < a.N;
-    const int32_t bias_n = (a.bias && n_ok) ? a.bias[n] : 0;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t m = m_base + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (n_ok && m < a.M) {
-          int32_t v = acc[i][j][r] + bias_n;
-          if (a.row_term)
-            v += a.row_term[m];
-          if (a.do_relu) {
-            v = v > 0 ? v : 0;
-            if (a.relu_limit > 0 && v > a.relu_limit)
-              v = (int32_t)a.relu_limit;
-          }
-          const int64_t o = m * a.N + n;
-          if (a.acc_out)
-            a.acc_out[o] = v;
-          if (a.has_rq)
-            store_out(a.out, o, requant_one(v, n, a.rq), a.rq.out_dtype);
-          else if (a.out)
-            ((int32_t *)a.out)[o] = v;
-        }
-      }
-    }
-  }
-}
 
 // ------------------------------------------------------------------------------------------------
 // Large-tile kernel: 256x256 outputs per workgroup, 8 waves (2 x 4, two per SIMD so that one wave's waits run under
@@ -341,6 +266,10 @@ __device__ __forceinline__ int32_t rshift_half_away_32(int32_t t, int32_t half, 
 // quarter of its tile, for shapes that would leave most CUs without a 256x256 tile.  Three stages of loads are in
 // flight while one is computed, so a short K loop costs about one memory latency, not one per step.
 // Requires K % 64 == 0; rows past M/N are clamped on the way in and masked on the way out.
+// ZP: operands with zero points, or unsigned ones.  Bytes are re-biased and summed in registers, on the fragments that
+// are multiplied anyway (8 vector instructions per fragment beside its share of a 16-pass MFMA): no pass over the
+// operands, no kernel for the sums and none to fold them into the bias (17 us of kernels and three launches at
+// 333 x 3000 x 1000 before).
 // ------------------------------------------------------------------------------------------------
 constexpr int MID_M = 128, MID_N = 128, MID_K = 64;
 // bt = tile edge: 128, or 64 (4 waves x one 32x32 block) for grids that would leave half the CUs without a 128-tile:
@@ -355,7 +284,7 @@ constexpr int mid_lds_bytes(int nst, int bt = 128) {
 
 // MID_NST = stages in the LDS ring: 4 (two workgroups per CU) when there are more tiles than CUs, 8 when every
 // workgroup has a CU to itself -- a short grid is bound by the bytes it keeps in flight.
-template <int MID_NST, int BT = 128>
+template <int MID_NST, int BT, bool ZP>
 __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m, int tiles_n, int per_xcd) {
   constexpr int WT = BT / 2;                       // a wave's square of outputs: 64 or 32
   constexpr int NB = WT / 32;                      // 32x32 MFMA blocks per side of it
@@ -456,6 +385,10 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
     }
   };
   load16(a.bias, 0, p_bias);
+  int32_t sum_a[NB], sum_b[NB];  // ZP: this lane's half of the sum of row i * 32 + lane % 32 of either operand
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+    sum_a[i] = sum_b[i] = 0;
   if (a.q31_half_away) {
     load16(a.rq.mult, a.rq.mult_s, p_mult);
     load16(a.rq.shift, a.rq.shift_s, p_shift);
@@ -477,6 +410,15 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
       for (int i = 0; i < NB; ++i) {
         fa[i] = *(const i32x4 *)(st + a_off[i] + (((ks * 2 + kh) ^ f_sw[i]) << 4));
         fb[i] = *(const i32x4 *)(st + b_off[i] + (((ks * 2 + kh) ^ f_sw[i]) << 4));
+        if constexpr (ZP) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            fa[i][e] ^= (int)a.a_flip4;
+            fb[i][e] ^= (int)a.b_flip4;
+          }
+          sum_a[i] = sum_bytes(__builtin_bit_cast(u32x4, fa[i]), sum_a[i]);
+          sum_b[i] = sum_bytes(__builtin_bit_cast(u32x4, fb[i]), sum_b[i]);
+        }
       }
 #pragma unroll
       for (int i = 0; i < NB; ++i)
@@ -491,6 +433,30 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
   // block) pass through a per-wave 64 x 64 strip in LDS so that a lane owns 16 consecutive columns of a row: per-column
   // parameters are loaded once per lane, and int8 results leave as 16-byte stores.
   __builtin_amdgcn_s_barrier();  // every wave is done reading the ring
+  if constexpr (ZP) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {  // lane l: column l % 32 of block column j, both k halves
+      const int32_t col = a.kzz - a.izp * (sum_b[j] + __shfl_xor(sum_b[j], 32, 64));
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          acc[i][j][r] += col;
+    }
+    if (a.rzp != 0) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int32_t rows = a.rzp * (sum_a[i] + __shfl_xor(sum_a[i], 32, 64));
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int32_t t = __shfl(rows, 8 * (r >> 2) + 4 * kh + (r & 3), 64);
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+            acc[i][j][r] -= t;
+        }
+      }
+    }
+  }
   int32_t *strip = (int32_t *)lds + wave * (WT * MID_STRIDE);
 #pragma unroll
   for (int i = 0; i < NB; ++i)
@@ -505,9 +471,10 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       p_half[e] = 1 << (p_shift[e] - 1);
-      p_zp[e] += 128;  // saturate as unsigned, flip the sign bits after
+      p_zp[e] += a.out_u8 ? 0 : 128;  // int8: saturate as unsigned, flip the sign bits after
     }
   }
+  const uint32_t out_flip4 = a.out_u8 ? 0u : 0x80808080u;
 #pragma unroll 1
   for (int it = 0; it < PASSES; ++it) {
     const int row = it * RPP + rsub;
@@ -520,12 +487,6 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
       v[q4 * 4 + 1] = t[1] + p_bias[q4 * 4 + 1];
       v[q4 * 4 + 2] = t[2] + p_bias[q4 * 4 + 2];
       v[q4 * 4 + 3] = t[3] + p_bias[q4 * 4 + 3];
-    }
-    if (a.row_term) {  // per-row term of a nonzero right zero point
-      const int32_t rt = a.row_term[m < a.M ? m : a.M - 1];
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        v[e] += rt;
     }
     if (a.do_relu) {
 #pragma unroll
@@ -559,7 +520,7 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
           const int32_t t = (int32_t)(p >> 31);
           q[u] = rshift_half_away_32(t, p_half[e], p_shift[e]) + p_zp[e];
         }
-        packed[q4] = sat_pack_u8(q[0], q[1], q[2], q[3]) ^ 0x80808080u;
+        packed[q4] = sat_pack_u8(q[0], q[1], q[2], q[3]) ^ out_flip4;
       }
       if (live) {
         int8_t *out = (int8_t *)a.out;
@@ -778,7 +739,7 @@ __global__ __launch_bounds__(512, 1) void i8_gemm_large_kernel(I8Args a, int til
       p_mult[e] = a.rq.mult ? a.rq.mult[n] : a.rq.mult_s;
       p_shift[e] = a.rq.shift ? a.rq.shift[n] : a.rq.shift_s;
       p_half[e] = 1 << (p_shift[e] - 1);
-      p_zp[e] = (a.rq.zp ? a.rq.zp[n] : a.rq.zp_s) + 128;  // +128: saturate as unsigned, flip the sign bits after
+      p_zp[e] = (a.rq.zp ? a.rq.zp[n] : a.rq.zp_s) + (a.out_u8 ? 0 : 128);  // int8: saturate as unsigned, flip the sign bits after
     }
   }
   // The short form of the Q31 requantization: with every accumulator below 2^30 in magnitude (small biases, K up to
@@ -786,7 +747,7 @@ __global__ __launch_bounds__(512, 1) void i8_gemm_large_kernel(I8Args a, int til
   // int32, so the rounding shift is an add and an arithmetic shift; with a zero output zero point the saturation is
   // one clamp and the bytes are picked by two permutes.  The workgroup-uniform conditions are tested here, the
   // bias one per wave.
-  const bool short_form = EPI == EPI_Q31_HALF_AWAY && !a.row_term && !a.do_relu && !a.acc_out && a.K <= 32768 &&
+  const bool short_form = EPI == EPI_Q31_HALF_AWAY && !a.out_u8 && !a.row_term && !a.do_relu && !a.acc_out && a.K <= 32768 &&
                           !a.rq.zp && a.rq.zp_s == 0 && __builtin_amdgcn_ballot_w64(!small_bias) == 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -894,7 +855,7 @@ __global__ __launch_bounds__(512, 1) void i8_gemm_large_kernel(I8Args a, int til
             const int32_t t = (int32_t)(p >> 31);
             q[u] = rshift_half_away_32(t, p_half[e], p_shift[e]) + p_zp[e];
           }
-          packed[q4] = sat_pack_u8(q[0], q[1], q[2], q[3]) ^ 0x80808080u;
+          packed[q4] = sat_pack_u8(q[0], q[1], q[2], q[3]) ^ (a.out_u8 ? 0u : 0x80808080u);
         }
         if (live) {
           int8_t *out = (int8_t *)a.out;
@@ -934,6 +895,8 @@ __device__ __forceinline__ u32x4 i8_load16_untracked(const void *p) {
   asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(v) : "v"(p) : "memory");
   return v;
 }
+// ZP: as in the mid-size kernel; a wave folds the sums of its own tiles into its own partial block.
+template <bool ZP>
 __global__ __launch_bounds__(512) void i8_rows32_kernel(I8Args a) {
   constexpr int WAVES = 8;
   constexpr int RING_BYTES = WAVES * 2 * 4096;  // per wave: two tiles of 32 rows x 128 bytes of the right operand
@@ -958,7 +921,7 @@ __global__ __launch_bounds__(512) void i8_rows32_kernel(I8Args a) {
   }
   uint8_t *ring = smem + wave * 8192;
   const uint8_t *bfrag = ring + c32 * 128;
-  const uint32_t fa = (uint32_t)a.a_flip * 0x01010101u, fb = (uint32_t)a.b_flip * 0x01010101u;
+  int32_t sum_a = 0, sum_b = 0;  // ZP: this lane's half of row / column lane % 32
   const int k_tiles = (int)(a.K / 128);
   // this wave's tiles: first, first + stride, ... (the waves of all K parts of the block take the tiles round-robin)
   const int first = part * WAVES + wave, stride = WAVES << a.split_shift;
@@ -995,10 +958,14 @@ __global__ __launch_bounds__(512) void i8_rows32_kernel(I8Args a) {
         for (int j = 0; j < 4; ++j) {
           u32x4 va = xa[u][j];
           u32x4 vb = *(const u32x4 *)(bfrag + u * 4096 + (((4 * h + j) ^ ((c32 >> 1) & 7)) << 4));
+          if constexpr (ZP) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            va[e] ^= fa;
-            vb[e] ^= fb;
+            for (int e = 0; e < 4; ++e) {
+              va[e] ^= a.a_flip4;
+              vb[e] ^= a.b_flip4;
+            }
+            sum_a = sum_bytes(va, sum_a);
+            sum_b = sum_bytes(vb, sum_b);
           }
           acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, va), __builtin_bit_cast(i32x4, vb), acc,
                                                       0, 0, 0);
@@ -1011,6 +978,12 @@ __global__ __launch_bounds__(512) void i8_rows32_kernel(I8Args a) {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         asm volatile("" : "+v"(xa[u][j]));  // their registers stay taken until here
+  }
+  if constexpr (ZP) {
+    const int32_t col = a.izp * (sum_b + __shfl_xor(sum_b, 32, 64)), rows = a.rzp * (sum_a + __shfl_xor(sum_a, 32, 64));
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      acc[r] -= col + __shfl(rows, 8 * (r >> 2) + 4 * h + (r & 3), 64);
   }
   __syncthreads();  // the partial blocks overlay the rings: every wave is done with its tiles
   // cross-wave sum, in wave order.  Register r of lane l is row 8 * (r / 4) + 4 * (l / 32) + r % 4, column l % 32.
@@ -1059,9 +1032,7 @@ __global__ __launch_bounds__(512) void i8_rows32_kernel(I8Args a) {
     int32_t v = sum[q];
     const int64_t m = 8 * (r >> 2) + 4 * h + (r & 3);
     if (m < a.M && n < a.N) {
-      v += bias_n;
-      if (a.row_term)
-        v += a.row_term[m];
+      v += bias_n + a.kzz;
       if (a.do_relu) {
         v = v > 0 ? v : 0;
         if (a.relu_limit > 0 && v > a.relu_limit)
@@ -1123,50 +1094,25 @@ int i8mm_launch(const void *d_a, int a_unsigned, const void *d_b, int b_unsigned
     return MI_SUCCESS;
 
   // unsigned bytes become signed by flipping the top bit; the zero point moves with them
-  int64_t izp = input_zp - (a_unsigned ? 128 : 0);
-  int64_t rzp = right_zp - (b_unsigned ? 128 : 0);
-
-  uint8_t *bt = nullptr;
-  int32_t *colsum = nullptr, *rowsum = nullptr, *bias_eff = nullptr, *row_term = nullptr;
-  const uint8_t *B = (const uint8_t *)d_b;
-  if (!right_transpose) {
-    MI_HIP(hipMallocAsync((void **)&bt, (size_t)N * K, stream));
-    dim3 grid((unsigned)((N + 63) / 64), (unsigned)((K + 63) / 64));
-    transpose_bytes_kernel<<<grid, dim3(256), 0, stream>>>((const uint8_t *)d_b, bt, K, N);
-    B = bt;
-  }
-  const int32_t *bias_use = d_bias;
-  if (izp != 0 || rzp != 0) {
-    if (izp != 0) {
-      MI_HIP(hipMallocAsync((void **)&colsum, (size_t)N * 4, stream));
-      row_sums_kernel<<<dim3((unsigned)((N + 3) / 4)), dim3(256), 0, stream>>>(B, b_unsigned, colsum, N, K);
-    }
-    MI_HIP(hipMallocAsync((void **)&bias_eff, (size_t)N * 4, stream));
-    fold_bias_kernel<<<dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream>>>(
-        d_bias, colsum, bias_eff, N, izp, rzp, K, b_unsigned ? 128 * K : 0);
-    bias_use = bias_eff;
-    if (rzp != 0) {
-      MI_HIP(hipMallocAsync((void **)&rowsum, (size_t)M * 4, stream));
-      MI_HIP(hipMallocAsync((void **)&row_term, (size_t)M * 4, stream));
-      row_sums_kernel<<<dim3((unsigned)((M + 3) / 4)), dim3(256), 0, stream>>>((const uint8_t *)d_a, a_unsigned,
-                                                                                rowsum, M, K);
-      row_term_kernel<<<dim3((unsigned)((M + 255) / 256)), dim3(256), 0, stream>>>(rowsum, row_term, M, rzp,
-                                                                                    a_unsigned ? 128 * K : 0);
-    }
-  }
+  const int64_t izp = input_zp - (a_unsigned ? 128 : 0);
+  const int64_t rzp = right_zp - (b_unsigned ? 128 : 0);
+  const bool zp = izp != 0 || rzp != 0 || a_unsigned || b_unsigned;
 
   I8Args a;
   a.A = (const uint8_t *)d_a;
-  a.B = B;
-  a.bias = bias_use;
-  a.row_term = row_term;
+  a.B = (const uint8_t *)d_b;
+  a.bias = d_bias;
+  a.row_term = nullptr;
   a.out = d_out;
   a.acc_out = d_acc;
   a.M = M;
   a.K = K;
   a.N = N;
-  a.a_flip = a_unsigned ? 0x80 : 0;
-  a.b_flip = b_unsigned ? 0x80 : 0;
+  a.a_flip4 = a_unsigned ? 0x80808080u : 0;
+  a.b_flip4 = b_unsigned ? 0x80808080u : 0;
+  a.izp = (int32_t)izp;
+  a.rzp = (int32_t)rzp;
+  a.kzz = (int32_t)((uint64_t)K * (uint64_t)izp * (uint64_t)rzp);  // modulo 2^32, like the sums
   a.do_relu = do_relu;
   a.relu_limit = relu_limit;
   a.has_rq = rq != nullptr;
@@ -1182,20 +1128,21 @@ int i8mm_launch(const void *d_a, int a_unsigned, const void *d_b, int b_unsigned
     // without a synchronization, so such arrays take it only when the caller vouches for them in the descriptor.
     const bool shift_ok = rq->d_shift ? rq->per_channel_q31_checked != 0 : (rq->shift >= 1 && rq->shift <= 31);
     const bool mult_ok = rq->d_multiplier ? rq->per_channel_q31_checked != 0 : rq->multiplier != INT32_MIN;
-    epi = (q31 && rq->round_mode == MI_ROUND_HALF_AWAY_FROM_ZERO && rq->out_dtype == MI_DT_I8 && shift_ok && mult_ok)
+    epi = (q31 && rq->round_mode == MI_ROUND_HALF_AWAY_FROM_ZERO &&
+           (rq->out_dtype == MI_DT_I8 || rq->out_dtype == MI_DT_U8) && shift_ok && mult_ok)
               ? EPI_Q31_HALF_AWAY
               : EPI_GENERIC;
   }
   a.q31_half_away = epi == EPI_Q31_HALF_AWAY;
+  a.out_u8 = rq && rq->out_dtype == MI_DT_U8;
   if (rq)
     a.rq = make_rq(rq);
   else
     a.rq = RequantParams{nullptr, nullptr, nullptr, 1, 0, 0, MI_RQ_MULTIPLIER_SHIFT, 0, 0, MI_DT_I32, 1.0f};
-  // 256x256 tiles when there are enough of them to occupy the chip, else 128x128 tiles on the same data path; the
-  // register-staged kernel takes what is left (K % 64 != 0)
+  // 256x256 tiles when there are enough of them to occupy the chip, else 128x128 tiles on the same data path
   const int64_t tiles_large = ((M + LM - 1) / LM) * ((N + LN - 1) / LN);
-  const bool large_ok = (K % 128) == 0 && M >= 128 && N >= 128, mid_ok = (K % 64) == 0;
-  const int tile_pick = plan().i8_tile ? plan().i8_tile : (large_ok && tiles_large >= 144 ? 256 : 128);  // measured crossover
+  const bool large_ok = M >= 128 && N >= 128;
+  const int tile_pick = plan().i8_tile > 0 ? plan().i8_tile : (large_ok && tiles_large >= 144 ? 256 : 128);  // measured crossover
   // up to 32 rows: the streaming kernel (plan: i8_tile = 32 asks for it, any other value rules it out).  Every
   // workgroup of it reads all of the left operand, so it is taken where that is little beside its 32 columns of the
   // right one, or where the 64 x 64 tiles are too few and too long.  Measured, 64 x 64 tiles / this one in us (launches
@@ -1206,45 +1153,71 @@ int i8mm_launch(const void *d_a, int a_unsigned, const void *d_b, int b_unsigned
   const bool few_pays = M * N <= 45056 || (N <= 8192 && (M <= 24 || K > 4096));
   const bool few = few_fits && (plan().i8_tile == 32 || (plan().i8_tile == 0 && few_pays));
   const bool large = !few && large_ok && tile_pick == 256;
-  const bool mid = !few && !large && mid_ok && tile_pick > 0;
-  uint8_t *a_signed = nullptr, *b_signed = nullptr;
-  if (large || mid) {
-    // direct-to-LDS loads cannot flip sign bits on the way: unsigned operands are rewritten once (after the
-    // zero-point sums above, which read the original bytes)
-    if (a_unsigned) {
-      MI_HIP(hipMallocAsync((void **)&a_signed, (size_t)M * K, stream));
-      flip_bytes_kernel<<<dim3((unsigned)((M * K / 16 + 256) / 256)), dim3(256), 0, stream>>>(a.A, a_signed, M * K);
-      a.A = a_signed;
+
+  // What has to be rewritten first.  The large kernel takes K in pairs of stages and signed bytes only (its fragment
+  // registers leave no room to re-bias); the others take stages of 64 and re-bias as they go, so that their padding is
+  // the byte that re-biases to zero.
+  const int64_t Kp = few ? K : (K + (large ? 127 : 63)) / (large ? 128 : 64) * (large ? 128 : 64);
+  const bool rewrite_a = Kp != K || (large && a_unsigned);
+  const bool rewrite_b = Kp != K || (large && b_unsigned) || !right_transpose;
+  const bool fold = large && (izp != 0 || rzp != 0);
+  ScratchBytes scratch;
+  if (rewrite_a || rewrite_b || fold) {
+    auto up = [](int64_t v) { return (size_t)((v + 255) & ~(int64_t)255); };
+    const size_t a_bytes = rewrite_a ? up(M * Kp) : 0, b_bytes = rewrite_b ? up(N * Kp) : 0;
+    const size_t bias_bytes = fold ? up(N * 4) : 0, row_bytes = fold && rzp != 0 ? up(M * 4) : 0;
+    const int rc = scratch.get(stream, WS_I8_OPERANDS, a_bytes + b_bytes + bias_bytes + row_bytes);
+    if (rc != MI_SUCCESS)
+      return rc;
+    uint8_t *p = (uint8_t *)scratch.ptr;
+    I8Copy ca = {}, cb = {};
+    if (rewrite_a) {
+      ca = I8Copy{a.A, p, M, K, Kp, (M * (Kp / 16) + 255) / 256, 0, large ? a.a_flip4 : 0, large ? 0 : a.a_flip4};
+      a.A = p;
     }
-    if (b_unsigned) {
-      MI_HIP(hipMallocAsync((void **)&b_signed, (size_t)N * K, stream));
-      flip_bytes_kernel<<<dim3((unsigned)((N * K / 16 + 256) / 256)), dim3(256), 0, stream>>>(a.B, b_signed, N * K);
-      a.B = b_signed;
+    if (rewrite_b) {
+      cb = I8Copy{a.B, p + a_bytes, N, K, Kp, 0, !right_transpose, large ? a.b_flip4 : 0, large ? 0 : a.b_flip4};
+      cb.blocks = cb.transpose ? ((N + 127) / 128) * ((Kp + 127) / 128) : (N * (Kp / 16) + 255) / 256;
+      a.B = p + a_bytes;
     }
+    if (rewrite_a || rewrite_b) {
+      MI_REQUIRE(ca.blocks + cb.blocks < (1ll << 31), MI_BAD_ARGUMENT, "mi_i8mm_launch: operands too large");
+      i8_prepare_kernel<<<dim3((unsigned)(ca.blocks + cb.blocks)), dim3(256), 0, stream>>>(ca, cb);
+    }
+    if (fold) {
+      int32_t *bias_eff = (int32_t *)(p + a_bytes + b_bytes);
+      int32_t *row_term = rzp != 0 ? (int32_t *)(p + a_bytes + b_bytes + bias_bytes) : nullptr;
+      const int64_t rows = N + (row_term ? M : 0);
+      i8_zero_terms_kernel<<<dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream>>>(
+          a.A, a.B, M, N, Kp, a.izp, a.rzp, a.kzz, d_bias, bias_eff, row_term);
+      a.bias = bias_eff;
+      a.row_term = row_term;
+    }
+    a.K = Kp;
   }
-  if (mid) {
-    int tiles_m = (int)((M + MID_M - 1) / MID_M), tiles_n = (int)((N + MID_N - 1) / MID_N);
-    int per_xcd = (tiles_m * tiles_n + 7) / 8;
-    static LdsLimitOnce lim4, lim8, lim64;
-    lim4.ensure((const void *)i8_gemm_mid_kernel<4>, 160 * 1024);
-    lim8.ensure((const void *)i8_gemm_mid_kernel<8>, 160 * 1024);
-    lim64.ensure((const void *)i8_gemm_mid_kernel<4, 64>, 160 * 1024);
-    // up to 128 tiles of 128 x 128 (half the CUs): 64 x 64 tiles with a 4-stage ring, four workgroups per CU hiding
-    // each other's waits (measured against the 128-tile forms: 5.8 vs 10.2 us at 256 x 1024 x 1024, 6.2 vs 10.5 at
-    // 1024^3, 11.2 vs 15.4 at 1024 x 2048 x 2048; from 160 tiles on the 128-tile forms win)
-    const int ring = plan().i8_mid_ring ? plan().i8_mid_ring : (tiles_m * tiles_n <= 128 ? 64 : tiles_m * tiles_n <= 256 ? 8 : 4);
-    if (ring == 64) {
-      tiles_m = (int)((M + 63) / 64);
-      tiles_n = (int)((N + 63) / 64);
-      per_xcd = (tiles_m * tiles_n + 7) / 8;
-      i8_gemm_mid_kernel<4, 64><<<dim3((unsigned)(per_xcd * 8)), dim3(256), mid_lds_bytes(4, 64), stream>>>(
-          a, tiles_m, tiles_n, per_xcd);
-    } else if (ring == 8)
-      i8_gemm_mid_kernel<8><<<dim3((unsigned)(per_xcd * 8)), dim3(256), mid_lds_bytes(8), stream>>>(a, tiles_m, tiles_n,
-                                                                                                   per_xcd);
+  if (few) {
+    const int64_t blocks = (N + 31) / 32;
+    MI_REQUIRE(blocks < (1ll << 29), MI_BAD_ARGUMENT, "i8 matmul: too many output columns");
+    // K shared by 2 or 4 workgroups per block while the launch stays within one workgroup per CU and every wave keeps
+    // four tiles (4096 x 11008, 128 blocks on 256 CUs otherwise: M = 1 17.7 -> 16.3 us, M = 32 29.1 -> 21.7; with two
+    // tiles a wave, 4096 x 4096: 8.7 -> 9.6)
+    while (a.split_shift < 2 && (blocks << (a.split_shift + 1)) <= R32_SPLIT_MAX_WGS &&
+           K / 128 >= (32 << (a.split_shift + 1)))
+      ++a.split_shift;
+    if (a.split_shift != 0) {
+      void *p = nullptr;
+      const int rc = stream_workspace(stream, WS_ROWS32_SPLIT,
+                                      R32_SPLIT_COUNTER_BYTES + (size_t)R32_SPLIT_MAX_WGS * 4096, &p, /*zero_fresh=*/true);
+      if (rc != MI_SUCCESS)  // (a stream under capture that never ran such a shape: the caller runs it eagerly first)
+        return rc;
+      a.counters = (unsigned *)p;
+      a.part = (int32_t *)((uint8_t *)p + R32_SPLIT_COUNTER_BYTES);
+    }
+    const dim3 grid((unsigned)(blocks << a.split_shift));
+    if (zp)
+      i8_rows32_kernel<true><<<grid, dim3(512), 0, stream>>>(a);
     else
-      i8_gemm_mid_kernel<4><<<dim3((unsigned)(per_xcd * 8)), dim3(256), mid_lds_bytes(4), stream>>>(a, tiles_m, tiles_n,
-                                                                                                   per_xcd);
+      i8_rows32_kernel<false><<<grid, dim3(512), 0, stream>>>(a);
   } else if (large) {
     const int tiles_m = (int)((M + LM - 1) / LM), tiles_n = (int)((N + LN - 1) / LN);
     const int per_xcd = (tiles_m * tiles_n + 7) / 8;
@@ -1262,46 +1235,38 @@ int i8mm_launch(const void *d_a, int a_unsigned, const void *d_b, int b_unsigned
     else
       MI_LARGE(EPI_GENERIC)
 #undef MI_LARGE
-  } else if (few) {
-    const int64_t blocks = (N + 31) / 32;
-    MI_REQUIRE(blocks < (1ll << 29), MI_BAD_ARGUMENT, "i8 matmul: too many output columns");
-    // K shared by 2 or 4 workgroups per block while the launch stays within one workgroup per CU and every wave keeps
-    // four tiles (4096 x 11008, 128 blocks on 256 CUs otherwise: M = 1 17.7 -> 16.3 us, M = 32 29.1 -> 21.7; with two
-    // tiles a wave, 4096 x 4096: 8.7 -> 9.6)
-    a.split_shift = 0;
-    while (a.split_shift < 2 && (blocks << (a.split_shift + 1)) <= R32_SPLIT_MAX_WGS &&
-           K / 128 >= (32 << (a.split_shift + 1)))
-      ++a.split_shift;
-    if (a.split_shift != 0) {
-      void *p = nullptr;
-      const int rc = stream_workspace(stream, WS_ROWS32_SPLIT,
-                                      R32_SPLIT_COUNTER_BYTES + (size_t)R32_SPLIT_MAX_WGS * 4096, &p, /*zero_fresh=*/true);
-      if (rc != MI_SUCCESS)  // (a stream under capture that never ran such a shape: the caller runs it eagerly first)
-        return rc;
-      a.counters = (unsigned *)p;
-      a.part = (int32_t *)((uint8_t *)p + R32_SPLIT_COUNTER_BYTES);
-    }
-    i8_rows32_kernel<<<dim3((unsigned)(blocks << a.split_shift)), dim3(512), 0, stream>>>(a);
   } else {
-    dim3 grid((unsigned)((N + BN - 1) / BN), (unsigned)((M + BM - 1) / BM));
-    i8_gemm_kernel<<<grid, dim3(256), 0, stream>>>(a);
+    const int64_t tiles128 = ((M + MID_M - 1) / MID_M) * ((N + MID_N - 1) / MID_N);
+    // up to 128 tiles of 128 x 128 (half the CUs): 64 x 64 tiles with a 4-stage ring, four workgroups per CU hiding
+    // each other's waits (measured against the 128-tile forms: 5.8 vs 10.2 us at 256 x 1024 x 1024, 6.2 vs 10.5 at
+    // 1024^3, 11.2 vs 15.4 at 1024 x 2048 x 2048; from 160 tiles on the 128-tile forms win)
+    const int ring = plan().i8_mid_ring ? plan().i8_mid_ring : (tiles128 <= 128 ? 64 : tiles128 <= 256 ? 8 : 4);
+    const int bt = ring == 64 ? 64 : 128;
+    const int tiles_m = (int)((M + bt - 1) / bt), tiles_n = (int)((N + bt - 1) / bt);
+    const int per_xcd = (tiles_m * tiles_n + 7) / 8;
+    const dim3 grid((unsigned)(per_xcd * 8));
+#define MI_MID(NST, BT, ZP)                                                                                        \
+  {                                                                                                                \
+    static LdsLimitOnce lds_limit;                                                                                 \
+    lds_limit.ensure((const void *)i8_gemm_mid_kernel<NST, BT, ZP>, 160 * 1024);                                   \
+    i8_gemm_mid_kernel<NST, BT, ZP><<<grid, dim3(256), mid_lds_bytes(NST, BT), stream>>>(a, tiles_m, tiles_n, per_xcd); \
+  }
+    if (ring == 64 && zp)
+      MI_MID(4, 64, true)
+    else if (ring == 64)
+      MI_MID(4, 64, false)
+    else if (ring == 8 && zp)
+      MI_MID(8, 128, true)
+    else if (ring == 8)
+      MI_MID(8, 128, false)
+    else if (zp)
+      MI_MID(4, 128, true)
+    else
+      MI_MID(4, 128, false)
+#undef MI_MID
   }
   MI_HIP(hipGetLastError());
-  if (a_signed)
-    MI_HIP(hipFreeAsync(a_signed, stream));
-  if (b_signed)
-    MI_HIP(hipFreeAsync(b_signed, stream));
-  if (bt)
-    MI_HIP(hipFreeAsync(bt, stream));
-  if (colsum)
-    MI_HIP(hipFreeAsync(colsum, stream));
-  if (rowsum)
-    MI_HIP(hipFreeAsync(rowsum, stream));
-  if (bias_eff)
-    MI_HIP(hipFreeAsync(bias_eff, stream));
-  if (row_term)
-    MI_HIP(hipFreeAsync(row_term, stream));
-  return MI_SUCCESS;
+  return scratch.release();
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -22,7 +22,7 @@ typedef struct mi_internal_plan {
   int a16_gemm_splits;               // > 0: number of K splits of the tiled kernel
   int a16_gemm_tile;                 // 128 / 256: columns per output block
   int a16_gemm_rows;                 // 16 / 32 / 64 / 128: rows per output block
-  int i8_tile;                       // 256 / 128 / 32 (streaming kernel for up to 32 rows) / -1 (register-staged kernel)
+  int i8_tile;                       // 256 / 128 / 32 (streaming kernel for up to 32 rows) / -1 (the tile kernels' own choice, never the streaming one)
   int i8_mid_ring;                   // 4 / 8 (128-tiles), 64 (64-tiles)
   int i8_ring;                       // not read any more (the large kernel has one ring form); kept so that the record keeps its layout
   int dq_waves;                      // 8 / 16
@@ -172,7 +172,7 @@ int a16_launch_group(const mi_a16_weight *const *ws, int n, const uint16_t *d_x,
 
 // library-owned scratch, one buffer per (device, stream, purpose) (workspace.hip); contents are whatever the last
 // user left
-enum { WS_SPLIT_K = 0, WS_DYNAMIC_QUANT = 1, WS_F8_TRANSPOSE = 2, WS_ROWS32_SPLIT = 3 };
+enum { WS_SPLIT_K = 0, WS_DYNAMIC_QUANT = 1, WS_F8_TRANSPOSE = 2, WS_ROWS32_SPLIT = 3, WS_I8_OPERANDS = 4 };
 // WS_ROWS32_SPLIT, shared by the few-row kernels that split K over workgroups (A16 and INT8): arrival counters, then
 // one 32 x 32 block of partial sums per workgroup.  Always asked for at this one size, so it is never re-allocated.
 constexpr int R32_SPLIT_MAX_WGS = 256;          // workgroups of a split launch, at most
@@ -181,6 +181,18 @@ constexpr int R32_SPLIT_COUNTER_BYTES = 1024;   // one counter per block of a sp
 // for the same size)
 int stream_workspace(hipStream_t st, int purpose, size_t bytes, void **out, bool zero_fresh = false);
 long workspace_allocations();
+// Scratch of one launch that a stream under capture may also need, and whose size follows the caller's operands: up to
+// 64 MiB of the stream's buffer (sizes in powers of two, so that what growing retires stays below what is in use), and
+// beyond that, or where the buffer would have to grow under capture, memory of this launch alone from the runtime's
+// stream-ordered pool.  (That pool for every call, as it was: it gives its memory back at each synchronization and takes
+// about 60 us to get it again.)
+struct ScratchBytes {
+  void *ptr = nullptr;
+  bool own = false;
+  hipStream_t stream = nullptr;
+  int get(hipStream_t st, int purpose, size_t bytes);
+  int release();  // after the last launch that uses it
+};
 // frees every buffer of a stream (current and retired); for owners of private streams, right before hipStreamDestroy
 void release_stream_workspaces(hipStream_t st);
 

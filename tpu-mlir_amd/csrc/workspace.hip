@@ -58,6 +58,34 @@ int stream_workspace(hipStream_t st, int purpose, size_t bytes, void **out, bool
   return MI_SUCCESS;
 }
 
+int ScratchBytes::get(hipStream_t st, int purpose, size_t bytes) {
+  stream = st;
+  size_t want = 1 << 16;
+  while (want < bytes)
+    want *= 2;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  bool kept = want <= ((size_t)64 << 20);
+  if (kept && hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {
+    int dev = 0;
+    MI_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lock(g_mutex);
+    const auto it = g_bufs.find(std::make_tuple(dev, st, purpose));
+    kept = it != g_bufs.end() && it->second.bytes >= want;
+  }
+  if (kept)
+    return stream_workspace(st, purpose, want, &ptr);
+  MI_HIP(hipMallocAsync(&ptr, bytes, st));
+  own = true;
+  return MI_SUCCESS;
+}
+
+int ScratchBytes::release() {
+  if (own)
+    MI_HIP(hipFreeAsync(ptr, stream));
+  own = false;
+  return MI_SUCCESS;
+}
+
 long workspace_allocations() {
   std::lock_guard<std::mutex> lock(g_mutex);
   return g_allocations;
