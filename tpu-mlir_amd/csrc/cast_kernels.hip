@@ -1,7 +1,7 @@
 // tpu.Cast for gfx950: elementwise conversion between the storage types on either side of the quantized matmuls
 // (f32 / bf16 / f16 / int8 / uint8 / int16 / uint16 / int32), following lib/Dialect/Tpu/Interfaces/Common/Cast.cpp:38-200
-// with requant()/dequant() of lib/Support/CastUtils.cpp:15-46 (BM168x branches).  HBM-bound: one read and one write
-// per element, 16 elements per thread.
+// with requant()/dequant() of lib/Support/CastUtils.cpp:15-46 (BM168x branches).  One read and one write per element:
+// HBM-bound when large, one memory round trip when small.
 #include "device_math.h"
 #include "internal.h"
 
@@ -179,12 +179,75 @@ __device__ __forceinline__ float cast_one(float x, const CastArgs &a) {
   return x;
 }
 
+// four consecutive elements: one request of 4, 8 or 16 bytes whatever the tensor's alignment
+template <typename T>
+__device__ __forceinline__ void load4(const void *p, int64_t i, T (&v)[4]) {
+  __builtin_memcpy(v, (const T *)p + i, sizeof(v));
+}
+__device__ __forceinline__ void load4_as_float(const void *p, int64_t i, int t, float (&x)[4]) {
+  const int size = st_size(t);
+  uint32_t raw[4];
+  uint16_t r2[4];
+  uint8_t r1[4];
+  if (size == 4)
+    load4(p, i, raw);
+  else if (size == 2)
+    load4(p, i, r2);
+  else
+    load4(p, i, r1);
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    x[e] = size == 4 ? load_as_float(&raw[e], 0, t) : size == 2 ? load_as_float(&r2[e], 0, t) : load_as_float(&r1[e], 0, t);
+}
+__device__ __forceinline__ void store4_from_float(void *p, int64_t i, int t, const float (&v)[4]) {
+  const int size = st_size(t);
+  uint32_t raw[4];
+  uint16_t r2[4];
+  uint8_t r1[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (size == 4)
+      store_from_float(&raw[e], 0, t, v[e]);
+    else if (size == 2)
+      store_from_float(&r2[e], 0, t, v[e]);
+    else
+      store_from_float(&r1[e], 0, t, v[e]);
+  }
+  if (size == 4)
+    __builtin_memcpy((uint32_t *)p + i, raw, sizeof(raw));
+  else if (size == 2)
+    __builtin_memcpy((uint16_t *)p + i, r2, sizeof(r2));
+  else
+    __builtin_memcpy((uint8_t *)p + i, r1, sizeof(r1));
+}
+
+// A thread takes four consecutive elements, so that a wave's requests are whole cache lines for every element size and
+// a small tensor is spread over as many workgroups as it has quarter kilobytes.  One element at a time, eight per
+// thread, it took 9.4 us for 333000 float32 -> int8 and 7.5 us for 4096 float32 -> bf16; this way 4.0 and 2.2.
+// IN, OUT: storage types known at compile time, so that the choice of the branch above costs nothing; -1: any, from
+// the arguments.
+template <int IN, int OUT>
 __global__ __launch_bounds__(256) void cast_kernel(CastArgs a) {
-  const int64_t base = ((int64_t)blockIdx.x * 256 + threadIdx.x);
-  const int64_t stride = (int64_t)gridDim.x * 256;
-  for (int64_t i = base; i < a.n; i += stride) {  // consecutive lanes touch consecutive elements
-    const float x = load_as_float(a.in, i, a.f32_io ? MI_ST_F32 : a.in_type);
-    store_from_float(a.out, i, a.f32_io ? MI_ST_F32 : a.out_type, cast_one(x, a));
+  if constexpr (IN >= 0) {
+    a.in_type = IN;
+    a.out_type = OUT;
+    a.f32_io = 0;
+    a.chip = MI_CHIP_BM168X;
+  }
+  const int in_t = a.f32_io ? MI_ST_F32 : a.in_type, out_t = a.f32_io ? MI_ST_F32 : a.out_type;
+  const int64_t stride = (int64_t)gridDim.x * 1024;
+  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4; i < a.n; i += stride) {
+    if (i + 4 <= a.n) {
+      float x[4];
+      load4_as_float(a.in, i, in_t, x);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        x[e] = cast_one(x[e], a);
+      store4_from_float(a.out, i, out_t, x);
+    } else {
+      for (int64_t k = i; k < a.n; ++k)
+        store_from_float(a.out, k, out_t, cast_one(load_as_float(a.in, k, in_t), a));
+    }
   }
 }
 
@@ -207,10 +270,27 @@ int cast_launch(const mi_cast_attr *c, const void *d_in, void *d_out, int64_t n,
   a.scale = scale;
   a.zero_point = (float)c->zero_point;
   a.chip = c->chip;
-  int64_t blocks = (n + 256 * 8 - 1) / (256 * 8);
-  if (blocks > 256 * 32)
+  int64_t blocks = (n + 1023) / 1024;
+  if (blocks > 256 * 32)  // eight rounds of 2048-thread CUs, then the loop
     blocks = 256 * 32;
-  cast_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(a);
+  const dim3 grid((unsigned)blocks);
+  const bool plain = !a.f32_io && a.chip != MI_CHIP_CV18XX;  // the chip model and the float-expanded view stay generic
+  auto is = [&](int in, int out) { return plain && a.in_type == in && a.out_type == out; };
+#define MI_CAST(IN, OUT)                                          \
+  if (is(IN, OUT))                                                \
+    cast_kernel<IN, OUT><<<grid, dim3(256), 0, stream>>>(a);      \
+  else
+  // the conversions on either side of the matmuls
+  MI_CAST(MI_ST_F32, MI_ST_BF16)
+  MI_CAST(MI_ST_BF16, MI_ST_F32)
+  MI_CAST(MI_ST_F32, MI_ST_F16)
+  MI_CAST(MI_ST_F16, MI_ST_F32)
+  MI_CAST(MI_ST_F32, MI_ST_I8)
+  MI_CAST(MI_ST_I8, MI_ST_F32)
+  MI_CAST(MI_ST_BF16, MI_ST_I8)
+  MI_CAST(MI_ST_I8, MI_ST_BF16)
+  cast_kernel<-1, -1><<<grid, dim3(256), 0, stream>>>(a);
+#undef MI_CAST
   MI_HIP(hipGetLastError());
   return MI_SUCCESS;
 }
