@@ -64,9 +64,9 @@ int permute_launch(const void *d_src, void *d_dst, int elem_bytes, int mode, int
 // right operand becomes [N, K], a K that is not a whole number of K stages is padded to one, and (for the kernel that
 // cannot do it on the way to the matrix cores) unsigned bytes are re-biased to signed.  HBM / launch bound: every
 // byte is read and written once, in 16-byte pieces whatever the row alignment (a piece that would reach past its row
-// is put together from bytes).  1000 x 3000 transposed + 333 x 1000 padded: 7.4 us, both operands; the 64 x 64
+// is put together from bytes).  1000 x 3000 transposed + 333 x 1000 padded: 6.4 us, both operands; the 64 x 64
 // byte-wise transpose it replaces took 10 us for the right operand alone, and the register-staged kernel that took any
-// K without padding 182 us for that product where the ring kernel below takes 14 (437 us at 333 x 1000 x 3000, now 18).
+// K without padding 182 us for that product where the ring kernel below takes 8.3 (437 us at 333 x 3000 x 1000, now 15.5).
 // ------------------------------------------------------------------------------------------------
 struct I8Copy {
   const uint8_t *src;
@@ -78,12 +78,29 @@ struct I8Copy {
   uint32_t pad4;       // what k >= K holds
 };
 
-// 16 bytes of a row of `len` bytes from position `at`: bytes past the end are `pad`
+// 16 bytes of a row of `len` bytes from position `at`: bytes past the end are `pad`.  The last piece of a row is the
+// row's last 16 bytes shifted into place, so that it costs one request like any other; only a row shorter than that is
+// read byte by byte.
 __device__ __forceinline__ u32x4 load16_ragged(const uint8_t *row, int64_t at, int64_t len, uint32_t pad4) {
   u32x4 v = {pad4, pad4, pad4, pad4};
-  if (at + 16 <= len) {
+  const int64_t over = at + 16 - len;
+  if (over <= 0) {
     __builtin_memcpy(&v, row + at, 16);
-  } else if (at < len) {
+  } else if (over < 16 && len >= 16) {
+    uint64_t q[2];
+    __builtin_memcpy(q, row + len - 16, 16);
+    const uint64_t pad8 = ((uint64_t)pad4 << 32) | pad4;
+    const int s = (int)(over & 7) * 8;  // pad4 is one byte repeated: whole words of it shift in from above
+    if (over >= 8) {
+      q[0] = q[1];
+      q[1] = pad8;
+    }
+    if (s) {
+      q[0] = (q[0] >> s) | (q[1] << (64 - s));
+      q[1] = (q[1] >> s) | (pad8 << (64 - s));
+    }
+    v = u32x4{(uint32_t)q[0], (uint32_t)(q[0] >> 32), (uint32_t)q[1], (uint32_t)(q[1] >> 32)};
+  } else if (over < 16) {
     uint32_t w[4] = {pad4, pad4, pad4, pad4};
     for (int i = 0; i < 16 && at + i < len; ++i) {
       const int sh = 8 * (i & 3);
@@ -92,6 +109,13 @@ __device__ __forceinline__ u32x4 load16_ragged(const uint8_t *row, int64_t at, i
     v = u32x4{w[0], w[1], w[2], w[3]};
   }
   return v;
+}
+
+// 16 bytes to any address
+template <typename V>
+__device__ __forceinline__ void store16(void *p, V v) {
+  static_assert(sizeof(V) == 16, "16 bytes");
+  __builtin_memcpy(p, &v, 16);
 }
 
 __device__ __forceinline__ void copy_rows(const I8Copy &c, int64_t block) {
@@ -359,11 +383,13 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
   // them before the epilogue
   const int cc = lane % CPR, rsub = lane / CPR;  // 16-column chunk, row within a group of RPP rows
   const int64_t n0 = n_base + wn * WT + cc * 16;
-  const bool vec_ok = (a.N % 16) == 0 && n0 + 16 <= a.N;
+  // whole: 16-byte accesses, of output rows at any alignment (element by element wherever N % 16 != 0, 333 x 1000 x 3000
+  // took 14.4 us; this way 8.3)
+  const bool vec_ok = n0 + 16 <= a.N;
   const int32_t relu_hi = (a.relu_limit > 0 && a.relu_limit < INT32_MAX) ? (int32_t)a.relu_limit : INT32_MAX;
   int32_t p_bias[16], p_mult[16], p_shift[16], p_zp[16];
-  // one array -> 16 registers: four 16-byte loads when the lane's columns are whole and aligned (the arrays are
-  // device allocations and n0 is a multiple of 16), else element by element with the index clamped
+  // one array -> 16 registers: four 16-byte loads when the lane's columns are whole (n0 is a multiple of 16), else
+  // element by element with the index clamped
   auto load16 = [&](const int32_t *src, int32_t dflt, int32_t (&dst)[16]) {
     if (!src) {
 #pragma unroll
@@ -499,7 +525,7 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
       if (vec_ok) {
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4)
-          *(i32x4 *)(a.acc_out + o + q4 * 4) = i32x4{v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3]};
+          store16(a.acc_out + o + q4 * 4, i32x4{v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3]});
       } else {
         for (int e = 0; e < 16; ++e)
           if (n0 + e < a.N)
@@ -525,7 +551,7 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
       if (live) {
         int8_t *out = (int8_t *)a.out;
         if (vec_ok) {
-          *(u32x4 *)(out + o) = u32x4{packed[0], packed[1], packed[2], packed[3]};
+          store16(out + o, u32x4{packed[0], packed[1], packed[2], packed[3]});
         } else {
           for (int e = 0; e < 16; ++e)
             if (n0 + e < a.N)
@@ -542,7 +568,7 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
       if (vec_ok) {
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4)
-          *(i32x4 *)(out + o + q4 * 4) = i32x4{v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3]};
+          store16(out + o + q4 * 4, i32x4{v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3]});
       } else {
         for (int e = 0; e < 16; ++e)
           if (n0 + e < a.N)
@@ -728,7 +754,7 @@ __global__ __launch_bounds__(512, 1) void i8_gemm_large_kernel(I8Args a, int til
   int32_t *strip = reinterpret_cast<int32_t *>(lds) + wave * (32 * SS);
   const int cc = lane & 3, rsub = lane >> 2;  // column chunk (16 columns) and row within a group of 16 rows
   const int64_t n0 = n_base + wn * 64 + cc * 16;
-  const bool vec_ok = (a.N % 16) == 0 && n0 + 16 <= a.N;
+  const bool vec_ok = n0 + 16 <= a.N;  // whole: 16-byte stores, of rows at any alignment
   // relu (and its optional upper limit) is one clamp, applied only when asked for
   const int32_t relu_hi = (a.relu_limit > 0 && a.relu_limit < INT32_MAX) ? (int32_t)a.relu_limit : INT32_MAX;
   int32_t p_mult[16], p_half[16], p_shift[16], p_zp[16];
@@ -793,7 +819,7 @@ __global__ __launch_bounds__(512, 1) void i8_gemm_large_kernel(I8Args a, int til
           if (live) {
             int8_t *out = (int8_t *)a.out;
             if (vec_ok) {
-              *(u32x4 *)(out + o) = u32x4{packed[0], packed[1], packed[2], packed[3]};
+              store16(out + o, u32x4{packed[0], packed[1], packed[2], packed[3]});
             } else {
               for (int e = 0; e < 16; ++e)
                 if (n0 + e < a.N)
@@ -818,7 +844,7 @@ __global__ __launch_bounds__(512, 1) void i8_gemm_large_kernel(I8Args a, int til
         if (vec_ok) {
 #pragma unroll
           for (int q4 = 0; q4 < 4; ++q4)
-            *(i32x4 *)(a.acc_out + o + q4 * 4) = i32x4{v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3]};
+            store16(a.acc_out + o + q4 * 4, i32x4{v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3]});
         } else {
           for (int e = 0; e < 16; ++e)
             if (n0 + e < a.N)
@@ -831,7 +857,7 @@ __global__ __launch_bounds__(512, 1) void i8_gemm_large_kernel(I8Args a, int til
           if (vec_ok) {
 #pragma unroll
             for (int q4 = 0; q4 < 4; ++q4)
-              *(i32x4 *)(out + o + q4 * 4) = i32x4{v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3]};
+              store16(out + o + q4 * 4, i32x4{v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3]});
           } else {
             for (int e = 0; e < 16; ++e)
               if (n0 + e < a.N)
@@ -860,7 +886,7 @@ __global__ __launch_bounds__(512, 1) void i8_gemm_large_kernel(I8Args a, int til
         if (live) {
           int8_t *out = (int8_t *)a.out;
           if (vec_ok) {
-            *(u32x4 *)(out + o) = u32x4{packed[0], packed[1], packed[2], packed[3]};
+            store16(out + o, u32x4{packed[0], packed[1], packed[2], packed[3]});
           } else {
             for (int e = 0; e < 16; ++e)
               if (n0 + e < a.N)
