@@ -487,3 +487,64 @@ def test_matmul_dynamic_f8_exact_domain_and_operator_level(orc):
         y = M_.matmul_dq(lf, rf, q_group_size=g, dq_type=getattr(clib, dq))
         w, _ = orc.matmul_dynamic(lf, rf, q_group_size=g, dq_type=getattr(orc, dq))
         assert np.array_equal(y, w)
+
+
+# ---- the tiled product (64 x 64 outputs per workgroup), forced at its edges -------------------------------------------
+TILE_CASES = [  # (bits, M, K, N, g, bias, dq): one to several tiles, ragged last ones; stages of one group, of several, of a part
+    (4, 1, 128, 16, 128, True, "INT"), (4, 63, 256, 65, 128, False, "INT"), (4, 65, 640, 129, 128, True, "INT"),
+    (4, 130, 512, 72, 64, True, "INT"), (4, 64, 384, 64, 32, True, "INT"), (4, 70, 1536, 100, 512, True, "INT"),
+    (8, 66, 384, 70, 128, True, "INT"), (8, 130, 256, 65, 64, False, "INT"), (8, 33, 128, 40, 32, True, "INT"),
+    (8, 65, 1024, 80, 256, True, "INT"), (4, 65, 384, 129, 128, True, "F4"), (4, 64, 256, 65, 64, False, "F4"),
+    (4, 66, 128, 33, 32, True, "F4"), (8, 65, 384, 129, 128, True, "F8"), (8, 70, 256, 64, 64, False, "F8"),
+    (8, 64, 128, 65, 32, True, "F8"),
+]
+
+
+@pytest.mark.parametrize("bits,M,K,N,g,bias,dq", TILE_CASES)
+def test_dynamic_tiles(orc, plan, bits, M, K, N, g, bias, dq):
+    plan(dq_waves=64)
+    if dq == "F8":
+        cfg = _f8_cfg(M, K, N, g, M + K, bias)
+    else:
+        cfg = S.w4a16(M, K, N, g, seed=M + K + N, bias=bias) if bits == 4 else S.w8a16(M, K, N, g, seed=M + K + N, bias=bias, signed=M % 2 == 0)
+        if bits == 8 and M % 2:
+            cfg["zp"] = np.random.default_rng(M).integers(0, 256, size=cfg["zp"].shape).astype(np.uint8)
+    out, pre = _device_typed(cfg, {"INT": clib.DQ_INT, "F4": clib.DQ_F4, "F8": clib.DQ_F8E4M3}[dq])
+    x, w, s, z, b = f32_valued_a16(cfg)
+    want, want_pre = orc.a16matmul_dynamic(x, w, s, z, b, M=M, K=K, N=N, weight_bits=bits, q_group_size=g,
+                                           dq_type={"INT": orc.DQ_INT, "F4": orc.DQ_F4, "F8": orc.DQ_F8E4M3}[dq])
+    if dq == "F8":  # group sums in the matrix core's order: 2^-20 of the terms' sum, far above what is seen
+        terms = np.abs(x).astype(np.float64) @ np.abs(_f8_weights(cfg)).T.astype(np.float64)
+        assert np.all(np.abs(pre - want_pre) <= 2.0 ** -20 * terms + 1e-30)
+    else:
+        assert np.array_equal(pre.view(np.uint32), want_pre.view(np.uint32))
+        assert np.array_equal(out, orc.f32_to_bf16(want))
+
+
+def _f8_weights(cfg):
+    """Dequantized E4M3 weights (|values| only matter here), scales per group applied."""
+    import torch
+    q = torch.from_numpy(cfg["weight"]).view(torch.float8_e4m3fn).float().numpy()
+    return q * np.repeat(S.bf16_to_f32(cfg["scale"]), cfg["g"], axis=1)
+
+
+@pytest.mark.parametrize("rt", [True, False])
+@pytest.mark.parametrize("M,K,N,g,dq", [(1, 64, 16, 64, "DQ_INT8"), (65, 128, 66, 64, "DQ_INT8"), (130, 192, 70, 64, "DQ_INT4"),
+                                        (64, 192, 129, 32, "DQ_INT8"), (63, 384, 65, 128, "DQ_INT8"), (66, 576, 40, 192, "DQ_INT4"),
+                                        (65, 256, 65, 32, "DQ_F4"), (70, 192, 64, 64, "DQ_F4")])
+def test_matmul_dynamic_tiles(orc, plan, M, K, N, g, dq, rt):
+    plan(dq_waves=64)
+    if dq.startswith("DQ_INT"):
+        test_matmul_dynamic_device_level(orc, M, K, N, g, rt, dq)
+        return
+    import torch
+    rng = np.random.default_rng(M + K + N)
+    lb = S.bf16_round(rng.standard_normal((M, K)).astype(np.float32))
+    rb = S.bf16_round(rng.standard_normal((N, K) if rt else (K, N)).astype(np.float32))
+    y32 = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    M_.matmul_dq_launch(torch.from_numpy(lb.view(np.int16)).cuda().view(torch.bfloat16),
+                        torch.from_numpy(rb.view(np.int16)).cuda().view(torch.bfloat16), right_transpose=rt, q_group_size=g,
+                        dq_type=getattr(clib, dq), y_f32=y32)
+    torch.cuda.synchronize()
+    _, want = orc.matmul_dynamic(S.bf16_to_f32(lb), S.bf16_to_f32(rb), right_transpose=rt, q_group_size=g, dq_type=getattr(orc, dq))
+    assert np.array_equal(y32.cpu().numpy().view(np.uint32), want.view(np.uint32))

@@ -6,13 +6,14 @@
 // group, and adds   isum * (amax / imax) * scale[n][g]   into the output in group order, the bias after the first
 // group.  Every piece of that is deterministic, so this path is bit-exact:
 //
-//   dq_act_kernel    one wave per (row, group): abs-max, the integer codes, their sum.  The codes are written straight
-//                    into the A-fragment order of v_mfma_i32_16x16x64_i8 that mirrors the packed weight tiles, so the
+//   dq_act_kernel    abs-max, the integer codes and their sum per row and group.  The codes are written straight into
+//                    the A-fragment order of v_mfma_i32_16x16x64_i8 that mirrors the packed weight tiles, so the
 //                    product kernel loads both operands with one coalesced 16-byte read per lane and never shuffles.
 //   dq_gemm_kernel   a workgroup owns 16 rows x 16 output channels; its waves take quantization groups round-robin,
 //                    each group an integer MFMA sum (nibbles 0..15 as int8, the zero point applied as zp * sum(codes)),
 //                    then the two fp32 multiplies of the reference; the per-group terms wait in LDS until 256 threads
-//                    add them up in group order.  Parallel over groups, sequential where the reference is.
+//                    add them up in group order.  Parallel over groups, sequential where the reference is.  For few
+//                    rows; from a few hundred outputs by a few hundred on, dq_tile.hip takes the product.
 //
 // The packed weight set is the one the static kernels read (a16_kernels.hip).  8-bit tiles hold unsigned bytes (int8
 // weights were flipped by 0x80 when packed) and, instead of an integer zero point, the exact float -(zp') * scale with
@@ -28,8 +29,7 @@
 //   F8E4M3  both operands widened to bf16 (exact) and multiplied on v_mfma_f32_16x16x32_bf16: the reference's group
 //           product is an f32 matmul whose summation order its library chooses, so parity is to fp32 rounding of the
 //           group sums; the fp8 instruction itself loses about 2^-14 of a sum to operand alignment and is not used.
-#include "a16_common.h"
-#include "internal.h"
+#include "dq_common.h"
 
 #include <type_traits>
 
@@ -37,107 +37,164 @@
 
 namespace mi {
 
-typedef __attribute__((ext_vector_type(4))) int i32x4;
-
-// dq_type families: integer codes (INT4 / INT8), E4M3 codes in 8-bit storage (F8E4M3), E2M1 codes in 4-bit storage (F4)
-constexpr int FLAV_INT = 0, FLAV_F8 = 1, FLAV_F4 = 2;
-
-// E2M1 magnitude codes are {0, .5, 1, 1.5, 2, 3, 4, 6}; as E4M3 bytes:
-constexpr uint32_t F4_AS_F8_LO = 0x3C383000u;  // 0, 0.5, 1, 1.5
-constexpr uint32_t F4_AS_F8_HI = 0x4C484440u;  // 2, 3, 4, 6
-__device__ __forceinline__ uint32_t f4_code_as_f8(uint32_t c) {
-  const uint32_t m = c & 7u;
-  const uint32_t tbl = m < 4 ? F4_AS_F8_LO : F4_AS_F8_HI;
-  return ((tbl >> (8 * (m & 3u))) & 0xffu) | ((c & 8u) << 4);
-}
-// four nibbles held one per byte (0..15 each) -> four E4M3 bytes
-__device__ __forceinline__ uint32_t f4x4_as_f8(uint32_t nib) {
-  return __builtin_amdgcn_perm(F4_AS_F8_HI, F4_AS_F8_LO, nib & 0x07070707u) | ((nib & 0x08080808u) << 4);
-}
-
 constexpr int DQ_WAVES = 8;
 constexpr int DQ_CHUNK = 128;  // groups whose terms fit the LDS buffer at once (1 KiB each)
 
-// position of element e (0..7) of a packed dword inside the 8 operand bytes it unpacks to: the low-nibble bytes of
-// the dword are elements 0,4,1,5 and the high-nibble bytes elements 2,6,3,7 (see unpack below)
-__device__ __forceinline__ int dq_slot(int e) { return ((e & 1) << 1) | ((e & 2) << 1) | (e >> 2); }
+// ---- activations -> codes in fragment order
+// aq: [m_blocks][K / 64][64 lanes][16 B]: lane (row, kq) of a 64-wide chunk holds k 8 kq .. + 8 in its low and
+// k 32 + 8 kq .. + 8 in its high eight bytes, in k order (8-bit layout) or in the slot order of an unpacked weight
+// dword (4-bit).  as_t / asum_t: [m_blocks][G][16 rows].
+//
+// A unit is 16 rows x one 64-wide chunk, or 16 rows x one group where groups are longer; 128 threads take it, eight
+// consecutive elements of a row and chunk each (one 16-byte load, one 8-byte store; the eight threads of a row meet
+// in three lane exchanges), so that a wave's stores are whole 128-byte pieces.  Memory- and latency-bound: 512 x 4096
+// took 10.5 us with a wave per row and group that stored its codes byte by byte, 5.6 us this way.
+// An operand stored [K][rows] (tpu.MatMul's usual right operand) is turned around through LDS on the way in.
+struct DqActJob {
+  const uint16_t *x;
+  uint8_t *aq;
+  float *as_t;
+  int32_t *asum_t;   // null: not wanted
+  int64_t rows, K;
+  int64_t units;     // m_blocks x (groups, or chunks where a chunk holds several groups); 0: no such operand
+  int transposed;
+};
 
-// ---- activations -> integer codes in fragment order
-// aq, 4-bit: [m_blocks][k_tiles of 128][2][64 lanes][16 B]; 8-bit: [m_blocks][k_tiles of 64][64 lanes][16 B] with byte
-// 8 h + e of lane (row, kq) = k 32 h + 8 kq + e of the tile.  as_t / asum_t: [m_blocks][G][16 rows]
 template <int DT, int BITS, int FLAV>
-__global__ __launch_bounds__(256) void dq_act_kernel(const uint16_t *__restrict__ x, int64_t M, int64_t K, int g, int G,
-                                                      float imax, int64_t k_tiles, uint8_t *__restrict__ aq,
-                                                      float *__restrict__ as_t, int32_t *__restrict__ asum_t,
-                                                      int64_t rows_padded) {
+__global__ __launch_bounds__(256) void dq_act_kernel(DqActJob ja, DqActJob jb, int g, int G, float imax) {
   using H = Half16<DT>;
-  const int lane = threadIdx.x & 63;
-  const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (wid >= rows_padded * G)
-    return;
-  const int64_t m = wid / G;
-  const int gi = (int)(wid - m * G);
-  const bool live = m < M;
-  // A16MatMul.cpp:98-108: amax starts at 1e-8
-  float amax = (float)1e-8;
-  if (live)
-    for (int k = lane; k < g; k += 64) {
-      const float v = fabsf(H::to_f32(x[m * K + (int64_t)gi * g + k]));
-      amax = amax > v ? amax : v;
-    }
+  __shared__ uint16_t turn[2][16][72];
+  const int t = threadIdx.x & 127, sub = threadIdx.x >> 7;
+  int64_t u = (int64_t)blockIdx.x * 2 + sub;
+  const bool second = u >= ja.units;
+  const DqActJob &j = second ? jb : ja;
+  if (second)
+    u -= ja.units;
+  const bool any = u < j.units;  // the last workgroup may have one unit only; it still meets the barriers
+  const int64_t per_block = g >= 64 ? G : j.K / 64;
+  const int64_t mb = any ? u / per_block : 0;
+  const int c0 = any ? (int)(u - mb * per_block) * (g >= 64 ? g / 64 : 1) : 0;  // first chunk of the unit
+  const int steps = g >= 64 ? g / 64 : 1;
+  const int row = t >> 3, l8 = t & 7;
+  const int64_t m = mb * 16 + row;
+  const bool live = any && m < j.rows;
+  const bool turns = ja.transposed || jb.transposed;  // the same for the whole workgroup: its barriers depend on it
+  auto load8 = [&](int step, uint16_t (&v)[8]) {
+    const int64_t k0 = (int64_t)(c0 + step) * 64;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
+    for (int e = 0; e < 8; ++e)
+      v[e] = 0;
+    if (live && !j.transposed)
+      __builtin_memcpy(v, j.x + m * j.K + k0 + l8 * 8, 16);
+    if (!turns)
+      return;
+    // thread t fetches row k0 + t / 2, eight columns of the block
+    const int64_t n = mb * 16 + (t & 1) * 8;
+    const uint16_t *src = j.x + (k0 + (t >> 1)) * j.rows + n;
+    uint16_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (any && j.transposed) {
+      if (n + 8 <= j.rows) {
+        __builtin_memcpy(w, src, 16);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (n + e < j.rows)
+            w[e] = src[e];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      turn[sub][(t & 1) * 8 + e][t >> 1] = w[e];
+    __syncthreads();
+    if (j.transposed) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        v[e] = turn[sub][row][l8 * 8 + e];
+    }
+  };
+  // A16MatMul.cpp:98-108: amax starts at 1e-8.  Two chunks stay in registers; longer groups are read a second time.
+  constexpr int HELD = 2;
+  uint16_t held[HELD][8];
+  float amax = (float)1e-8;
+  auto take_max = [&](const uint16_t (&v)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float f = fabsf(H::to_f32(v[e]));
+      amax = amax > f ? amax : f;
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < HELD; ++s)
+    if (s < steps) {
+      load8(s, held[s]);
+      take_max(held[s]);
+    }
+  for (int s = HELD; s < steps; ++s) {
+    uint16_t v[8];
+    load8(s, v);
+    take_max(v);
+  }
+  // the eight lanes of a row, or the four of its 32-wide group
+  const int lanes = g == 32 ? 4 : 8;
+  for (int o = lanes >> 1; o > 0; o >>= 1) {
     const float other = __shfl_xor(amax, o, 64);
     amax = amax > other ? amax : other;
   }
   // :109-132: integer types round(x / amax * imax), half away from zero; the float types round x / (amax / imax) to
   // their own grid, and the MFMA operand is that grid value's E4M3 byte (every E2M1 value is an E4M3 value)
+  const float step_size = amax / imax;
   int sum = 0;
   float fsum = 0.0f;
-  const float step = amax / imax;
-  const int64_t mb = m >> 4;
-  const int row = (int)(m & 15);
-  for (int k = lane; k < g; k += 64) {
-    const int64_t kk = (int64_t)gi * g + k;
-    int code = 0;
-    if (live) {
-      const float v = H::to_f32(x[m * K + kk]);
+  auto emit = [&](int step, const uint16_t (&v)[8]) {
+    uint32_t lo = 0, hi = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float f = H::to_f32(v[e]);
+      int code;
       if constexpr (FLAV == FLAV_INT) {
-        code = (int)roundf(v / amax * imax);
+        code = (int)roundf(f / amax * imax);
         sum += code;
       } else if constexpr (FLAV == FLAV_F8) {
         // F8E4M3(src, double step, true): the double quotient narrowed to f32 equals the f32 quotient (a quotient of
         // two f32 values never lies close enough to an f32 rounding boundary for the double rounding to matter)
-        code = (int)f8e4m3_from_f32(__fdiv_rn(v, step));
+        code = (int)f8e4m3_from_f32(__fdiv_rn(f, step_size));
         fsum += f8e4m3_to_f32((uint32_t)code);
       } else {
-        code = (int)f4_code_as_f8(f4e2m1_from_f32(__fdiv_rn(v, step)));
+        code = (int)f4_code_as_f8(f4e2m1_from_f32(__fdiv_rn(f, step_size)));
         fsum += f8e4m3_to_f32((uint32_t)code);
       }
+      const int at = BITS == 4 ? dq_slot(e) : e;
+      const uint32_t b = (uint32_t)(code & 0xff) << (8 * (at & 3));
+      if (at < 4)
+        lo |= b;
+      else
+        hi |= b;
     }
-    int64_t at;
-    if constexpr (BITS == 4) {
-      const int64_t kt = kk >> 7;
-      const int in_tile = (int)(kk & 127);
-      const int j = in_tile >> 5, kq = (in_tile >> 3) & 3, e = in_tile & 7;
-      at = ((((mb * k_tiles + kt) * 2 + (j >> 1)) * 64) + kq * 16 + row) * 16 + (j & 1) * 8 + dq_slot(e);
-    } else {
-      const int64_t kt = kk >> 6;
-      const int in_tile = (int)(kk & 63);
-      const int h = in_tile >> 5, kq = (in_tile >> 3) & 3, e = in_tile & 7;
-      at = (((mb * k_tiles + kt) * 64) + kq * 16 + row) * 16 + h * 8 + e;
-    }
-    aq[at] = (uint8_t)(int8_t)code;
-  }
+    if (!live)
+      lo = hi = 0;
+    if (any)
+      *(u32x2 *)(j.aq + (mb * (j.K / 64) + c0 + step) * 1024 + ((l8 & 3) * 16 + row) * 16 + (l8 >> 2) * 8) = u32x2{lo, hi};
+  };
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
+  for (int s = 0; s < HELD; ++s)
+    if (s < steps)
+      emit(s, held[s]);
+  for (int s = HELD; s < steps; ++s) {
+    uint16_t v[8];
+    load8(s, v);
+    emit(s, v);
+  }
+  for (int o = lanes >> 1; o > 0; o >>= 1) {
     sum += __shfl_xor(sum, o, 64);
     fsum += __shfl_xor(fsum, o, 64);
   }
-  if (lane == 0) {
+  if (any && (l8 & (lanes - 1)) == 0) {
+    const int64_t gi = g >= 64 ? u - mb * per_block : (int64_t)c0 * 2 + (l8 >> 2);
     const int64_t at = (mb * G + gi) * 16 + row;
-    as_t[at] = live ? step : 0.0f;  // :143-145 (cur_group_act_max[row] / imax)
-    asum_t[at] = FLAV == FLAV_INT ? sum : __float_as_int(fsum);  // what a nonzero weight zero point multiplies
+    j.as_t[at] = live ? step_size : 0.0f;  // :143-145 (cur_group_act_max[row] / imax)
+    if (j.asum_t)  // what a nonzero weight zero point multiplies
+      j.asum_t[at] = !live ? 0 : FLAV == FLAV_INT ? sum : __float_as_int(fsum);
   }
 }
 
@@ -160,28 +217,6 @@ struct DqArgs {
   int unit_groups;  // groups per unit: 1; 4-bit weights: 2 with g == 64, 4 with g == 32; 8-bit weights: 2 with g == 32
   int chip;
 };
-
-// nibbles of a packed dword as bytes: low nibbles (elements 0,4,1,5), high nibbles (elements 2,6,3,7)
-__device__ __forceinline__ void unpack_bytes(uint32_t d, int &lo, int &hi) {
-  lo = (int)(d & 0x0F0F0F0Fu);
-  hi = (int)((d >> 4) & 0x0F0F0F0Fu);
-}
-
-__device__ __forceinline__ long pack64(uint32_t lo, uint32_t hi) { return (long)(((uint64_t)hi << 32) | lo); }
-
-// eight E4M3 bytes -> eight bf16 values (exact: 4 significant bits into 8).  The fp8 matrix instructions align their
-// products to the largest one and drop low bits (about 2^-14 of the group sum here); the bf16 instruction fed with the
-// same values adds the exact products with fp32 rounding, which is what the reference's f32 matmul does.
-__device__ __forceinline__ bf16x8 f8x8_as_bf16(uint32_t lo, uint32_t hi) {
-  typedef __attribute__((ext_vector_type(2))) float f32x2;
-  const f32x2 p0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)lo, false), p1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)lo, true);
-  const f32x2 p2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hi, false), p3 = __builtin_amdgcn_cvt_pk_f32_fp8((int)hi, true);
-  const u32x4 r = {__builtin_amdgcn_perm(__float_as_uint(p0[1]), __float_as_uint(p0[0]), 0x07060302u),
-                   __builtin_amdgcn_perm(__float_as_uint(p1[1]), __float_as_uint(p1[0]), 0x07060302u),
-                   __builtin_amdgcn_perm(__float_as_uint(p2[1]), __float_as_uint(p2[0]), 0x07060302u),
-                   __builtin_amdgcn_perm(__float_as_uint(p3[1]), __float_as_uint(p3[0]), 0x07060302u)};
-  return __builtin_bit_cast(bf16x8, r);
-}
 
 // acc[which] += A x B on the fp8 instruction, which wave-uniform but not a compile-time constant: every accumulator
 // is named, so none of them is indexed
@@ -351,21 +386,19 @@ __global__ __launch_bounds__(2 * DQ_WAVES * 64) void dq_gemm_kernel(DqArgs a) {
 }
 
 // ---- tpu.MatMul with both operands quantized dynamically (lib/Dialect/Tpu/Interfaces/Common/MatMul.cpp:447-597,
-// integer dq types, batch 1).  Both operands go through dq_act_kernel (a [K, N] right operand is transposed first), and
+// integer dq types, batch 1).  Both operands go through dq_act_kernel in one launch, and
 // the product kernel is the one above with a second fragment stream in place of the weight tiles and the right
 // column's amax / imax in place of the weight scale.  The reference adds no bias and applies no relu on this branch.
-__global__ __launch_bounds__(256) void transpose16_kernel(const uint16_t *__restrict__ src, uint16_t *__restrict__ dst,
-                                                           int64_t rows, int64_t cols) {
-  __shared__ uint16_t tile[32][33];
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-  const int64_t c0 = (int64_t)blockIdx.x * 32, r0 = (int64_t)blockIdx.y * 32;
-  for (int i = ty; i < 32; i += 8)
-    if (r0 + i < rows && c0 + tx < cols)
-      tile[i][tx] = src[(r0 + i) * cols + c0 + tx];
-  __syncthreads();
-  for (int i = ty; i < 32; i += 8)
-    if (c0 + i < cols && r0 + tx < rows)
-      dst[(c0 + i) * rows + r0 + tx] = tile[tx][i];
+// Tiles of 64 x 64 outputs (dq_tile.hip), or blocks of 16 x 16 with K spread over the waves.  A tile walks K by itself
+// (12 us for 4096, however few there are); the blocks' time grows with their number.  Blocks / tiles in us, quantizer
+// included, W4 with groups of 128: 4096 x 4096 M = 64 (1024 blocks) 18.6 / 18.7, M = 128 26.3 / 19.5; N = 1024 M = 128
+// (512) 13.0 / 19.0, M = 512 28.8 / 21.2; N = 11008 M = 32 (1376) 20.4 / 19.6; K = 11008 M = 32 (512) 26.8 / 37.0,
+// M = 64 47.2 / 37.4; 2048 x 2048 groups of 64 M = 128 (1024) 15.8 / 17.9, M = 256 22.3 / 18.3; two activations
+// 512 x 512 (1024) K = 128 7.4 / 7.1, K = 1024 10.2 / 11.7; 1024 x 1024 13.7 / 7.6 and 22.2 / 14.1
+static bool dq_takes_tiles(int64_t m_blocks, int64_t n_blocks, int64_t K) {
+  if (plan().dq_waves)
+    return plan().dq_waves == 64;
+  return m_blocks * n_blocks >= (K >= 8192 ? 768 : 1280);
 }
 
 struct Dq2Args {
@@ -629,24 +662,19 @@ int matmul_dq_launch(const uint16_t *d_left, const uint16_t *d_right, int right_
   const int64_t m_blocks = (M + 15) / 16, n_blocks = (N + 15) / 16;
   const size_t al_bytes = (size_t)m_blocks * 16 * K, ar_bytes = (size_t)n_blocks * 16 * K;
   const size_t sl_bytes = (size_t)m_blocks * 16 * G * 4, sr_bytes = (size_t)n_blocks * 16 * G * 4;
-  const size_t tr_bytes = right_transpose ? 0 : (((size_t)N * K * 2 + 255) & ~(size_t)255);
   uint8_t *ws = nullptr;
-  int rc = stream_workspace(stream, WS_DYNAMIC_QUANT, tr_bytes + al_bytes + ar_bytes + 2 * (sl_bytes + sr_bytes),
-                            (void **)&ws);
+  int rc = stream_workspace(stream, WS_DYNAMIC_QUANT, al_bytes + ar_bytes + sl_bytes + sr_bytes, (void **)&ws);
   if (rc != MI_SUCCESS)
     return rc;
-  uint16_t *rt = (uint16_t *)ws;
-  uint8_t *aq_l = ws + tr_bytes, *aq_r = aq_l + al_bytes;
+  uint8_t *aq_l = ws, *aq_r = aq_l + al_bytes;
   float *as_l = (float *)(aq_r + ar_bytes), *as_r = as_l + sl_bytes / 4;
-  int32_t *sum_l = (int32_t *)(as_r + sr_bytes / 4), *sum_r = sum_l + sl_bytes / 4;  // written, not read
-  const uint16_t *right_nk = d_right;
-  if (!right_transpose) {
-    transpose16_kernel<<<dim3((unsigned)((N + 31) / 32), (unsigned)((K + 31) / 32)), dim3(256), 0, stream>>>(d_right, rt,
-                                                                                                        K, N);
-    right_nk = rt;
-  }
   const bool f16 = dtype == MI_DT_F16;
-  const int64_t wl = m_blocks * 16 * G, wr = n_blocks * 16 * G;
+  const int64_t per_block = g >= 64 ? G : k_tiles;
+  const DqActJob jl = {d_left, aq_l, as_l, nullptr, M, K, m_blocks * per_block, 0};
+  const DqActJob jr = {d_right, aq_r, as_r, nullptr, N, K, n_blocks * per_block, !right_transpose};
+  const dim3 act_grid((unsigned)((jl.units + jr.units + 1) / 2));
+  const int flavor = dq_type == MI_DQ_F8E4M3 ? FLAV_F8 : dq_type == MI_DQ_F4 ? FLAV_F4 : FLAV_INT;
+  const bool tiled = dq_takes_tiles(m_blocks, n_blocks, K);
   Dq2Args a;
   a.aq_l = (const u32x4 *)aq_l;
   a.aq_r = (const u32x4 *)aq_r;
@@ -666,13 +694,12 @@ int matmul_dq_launch(const uint16_t *d_left, const uint16_t *d_right, int right_
   // both operands in the 8-bit fragment layout, whatever the code type
 #define MI_DQ2_RUN(DT_, FLAV_)                                                                                  \
   {                                                                                                             \
-    dq_act_kernel<DT_, 8, FLAV_><<<dim3((unsigned)((wl + 3) / 4)), dim3(256), 0, stream>>>(                     \
-        d_left, M, K, (int)g, G, imax, k_tiles, aq_l, as_l, sum_l, m_blocks * 16);                              \
-    dq_act_kernel<DT_, 8, FLAV_><<<dim3((unsigned)((wr + 3) / 4)), dim3(256), 0, stream>>>(                     \
-        right_nk, N, K, (int)g, G, imax, k_tiles, aq_r, as_r, sum_r, n_blocks * 16);                            \
-    static LdsLimitOnce lds_limit;                                                                              \
-    lds_limit.ensure((const void *)dq2_gemm_kernel<DT_, FLAV_>, 160 * 1024);                                    \
-    dq2_gemm_kernel<DT_, FLAV_><<<grid, dim3(DQ_WAVES * 64), lds_bytes, stream>>>(a);                           \
+    dq_act_kernel<DT_, 8, FLAV_><<<act_grid, dim3(256), 0, stream>>>(jl, jr, (int)g, G, imax);                  \
+    if (!tiled) {                                                                                               \
+      static LdsLimitOnce lds_limit;                                                                            \
+      lds_limit.ensure((const void *)dq2_gemm_kernel<DT_, FLAV_>, 160 * 1024);                                  \
+      dq2_gemm_kernel<DT_, FLAV_><<<grid, dim3(DQ_WAVES * 64), lds_bytes, stream>>>(a);                         \
+    }                                                                                                           \
   }
   if (dq_type == MI_DQ_F8E4M3) {
     if (f16)
@@ -692,6 +719,11 @@ int matmul_dq_launch(const uint16_t *d_left, const uint16_t *d_right, int right_
   }
 #undef MI_DQ2_RUN
   MI_HIP(hipGetLastError());
+  if (tiled) {
+    const DqTileArgs ta = {aq_l, aq_r, as_l, nullptr, as_r, nullptr, nullptr, d_y, d_y32, M, N, (int)k_tiles, G, (int)g,
+                           dtype, MI_CHIP_BM168X};
+    return dq_tile_launch(ta, DQB_ACT, flavor, stream);
+  }
   return MI_SUCCESS;
 }
 
@@ -930,7 +962,10 @@ int a16_dq_launch(const mi_a16_weight *w, int dq_type, const uint16_t *d_x, int6
     return rc;
   float *as_t = (float *)(aq + aq_bytes);
   int32_t *asum_t = (int32_t *)(aq + aq_bytes + qp_bytes);
-  const int64_t waves = rows_padded * G;
+  const DqActJob job = {d_x, aq, as_t, asum_t, M, w->K, m_blocks * (g >= 64 ? G : w->K / 64), 0};
+  const DqActJob none = {};
+  const dim3 act_grid((unsigned)((job.units + 1) / 2));
+  const bool tiled = dq_takes_tiles(m_blocks, w->row_blocks, w->K);
   const bool f16 = w->dtype == MI_DT_F16;
   DqArgs a;
   a.qw = (const u32x4 *)w->qweight;
@@ -957,11 +992,12 @@ int a16_dq_launch(const mi_a16_weight *w, int dq_type, const uint16_t *d_x, int6
   const int gemm_waves = (wo == DQ_WAVES || wo == 2 * DQ_WAVES) ? wo : ((int64_t)w->row_blocks * m_blocks <= 256 ? 2 * DQ_WAVES : DQ_WAVES);
 #define MI_DQ_RUN(DT_, BITS_, FLAV_)                                                                             \
   {                                                                                                             \
-    dq_act_kernel<DT_, BITS_, FLAV_><<<dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream>>>(              \
-        d_x, M, w->K, g, G, imax, w->k_tiles, aq, as_t, asum_t, rows_padded);                                   \
-    static LdsLimitOnce lds_limit;                                                                              \
-    lds_limit.ensure((const void *)dq_gemm_kernel<DT_, BITS_, FLAV_>, 160 * 1024);                              \
-    dq_gemm_kernel<DT_, BITS_, FLAV_><<<grid, dim3(gemm_waves * 64), lds_bytes, stream>>>(a);                   \
+    dq_act_kernel<DT_, BITS_, FLAV_><<<act_grid, dim3(256), 0, stream>>>(job, none, g, G, imax);                \
+    if (!tiled) {                                                                                               \
+      static LdsLimitOnce lds_limit;                                                                            \
+      lds_limit.ensure((const void *)dq_gemm_kernel<DT_, BITS_, FLAV_>, 160 * 1024);                            \
+      dq_gemm_kernel<DT_, BITS_, FLAV_><<<grid, dim3(gemm_waves * 64), lds_bytes, stream>>>(a);                 \
+    }                                                                                                           \
   }
   if (dq_type == MI_DQ_F8E4M3) {
     if (f16)
@@ -986,6 +1022,12 @@ int a16_dq_launch(const mi_a16_weight *w, int dq_type, const uint16_t *d_x, int6
   }
 #undef MI_DQ_RUN
   MI_HIP(hipGetLastError());
+  if (tiled) {
+    const DqTileArgs ta = {aq, (const uint8_t *)w->qweight, as_t, asum_t, bits == 4 ? (const void *)w->sz_t : (const void *)w->scale_t,
+                           w->nzs_t, w->bias, d_y, d_y32, M, w->N, (int)(w->K / 64), G, g, w->dtype, w->chip};
+    const int flavor = dq_type == MI_DQ_F8E4M3 ? FLAV_F8 : dq_type == MI_DQ_F4 ? FLAV_F4 : FLAV_INT;
+    return dq_tile_launch(ta, bits == 4 ? DQB_W4 : DQB_W8, flavor, stream);
+  }
   return MI_SUCCESS;
 }
 

@@ -25,7 +25,7 @@ typedef struct mi_internal_plan {
   int i8_tile;                       // 256 / 128 / 32 (streaming kernel for up to 32 rows) / -1 (the tile kernels' own choice, never the streaming one)
   int i8_mid_ring;                   // 4 / 8 (128-tiles), 64 (64-tiles)
   int i8_ring;                       // not read any more (the large kernel has one ring form); kept so that the record keeps its layout
-  int dq_waves;                      // 8 / 16
+  int dq_waves;                      // 8 / 16 (16 x 16 blocks with that many waves), 64 (64 x 64 tiles)
   int f8_tile;                       // 256 / 128 / 64 / 32 (streaming kernel for up to 32 rows)
   int a16_decode_rows8;              // 1: five to eight rows always take the decode kernel where it can; -1: never
   int a16_rows32_min_m;              // > 0: sets it can handle take the 32-row kernel from this many rows (to 32); -1: never
