@@ -216,147 +216,226 @@ __device__ __forceinline__ void f8_epilogue(const F8Args &a, const f32x16 (&acc)
 
 // The reference's requantization is E4M3((float)((double)v / step)), Float8.cpp:259-261.  With inv an fp32 number within
 // 2^-23 of 1 / step (per channel: the scale itself rounded to fp32, since step = 1 / scale; one scale: fl32(1 / step)
-// from the host), q0 = v * inv is within 3.01 fp32 ulps of the real quotient v / step and the reference's fp32 quotient
-// within 0.51, so the two can only round to different E4M3 codes when a rounding boundary lies within 4 ulps of q0.
-// The test: q0 shrunk and grown
-// by 2^-20 (8 ulps or more) must convert to the same code; conversion is monotonic, so then every value in between
-// does, the reference's included.  Otherwise (about 6 outputs in 10^5) the division is carried out as written.  The
-// hardware conversion (v_cvt_pk_fp8_f32: round to nearest even, subnormals included) runs on values clamped to
-// +-448, which is the reference's saturation; NaN goes down the slow path.
-// the requantization as the reference writes it; out of line, so that the many unrolled call sites of the fast path
-// do not each carry a copy of two double divisions and the software conversion
-__device__ __attribute__((noinline)) uint32_t f8_requant_exact(float v, double step) {
-  return f8e4m3_from_f32((float)((double)v / step));
+// from the host), v * inv is within 3.01 fp32 ulps of the real quotient v / step and the reference's fp32 quotient
+// within 0.51, so the two can only round to different E4M3 codes when a rounding boundary lies within 4 ulps of v * inv.
+// The test: v times inv shrunk and grown by 2^-20 (7 ulps or more after their own roundings) must convert to the same
+// code; conversion is monotonic, so then every value in between does, the reference's included.  Otherwise (about 6
+// outputs in 10^5) the division is carried out as written, four outputs at a time.  The hardware conversion
+// (v_cvt_pk_fp8_f32: round to nearest even, subnormals included) runs on values clamped to +-448, which is the
+// reference's saturation; NaN goes down the slow path.
+// four columns' requantization as the reference writes it; out of line, so that the call sites of the fast path do not
+// each carry copies of the double divisions and the software conversion
+__device__ __attribute__((noinline)) uint32_t f8_requant_exact4(float v0, float v1, float v2, float v3, const double *scales,
+                                                                int64_t n, int64_t last, double step) {
+  const float v[4] = {v0, v1, v2, v3};
+  uint32_t w = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const double st = scales ? 1.0 / scales[n + e < last ? n + e : last] : step;
+    w |= f8e4m3_from_f32((float)((double)v[e] / st)) << (8 * e);
+  }
+  return w;
 }
 
-__device__ __forceinline__ uint32_t f8_requant_pair(const F8Args &a, float v0, float v1, float inv0, float inv1,
-                                                    int64_t n0, int64_t n1) {
-  const float q0 = __builtin_fminf(__builtin_fmaxf(v0 * inv0, -448.0f), 448.0f);
-  const float q1 = __builtin_fminf(__builtin_fmaxf(v1 * inv1, -448.0f), 448.0f);
+// what a lane keeps of the 16 consecutive columns it finishes
+struct F8Cols {
+  int64_t n0;
+  bool whole;                          // all 16 exist: 16-byte accesses, of output rows at any alignment
+  float bias[16], inv_lo[16], inv_hi[16];  // inv_lo / inv_hi: fl32(1 / step) shrunk / grown by 2^-20
+};
+__device__ __forceinline__ void f8_load_cols(const F8Args &a, F8Cols &c, int64_t n0) {
   constexpr float DN = 1.0f - 0x1p-20f, UP = 1.0f + 0x1p-20f;
-  const uint32_t mid = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(q0, q1, 0, false) & 0xffffu;
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(q0 * DN, q1 * DN, 0, false) & 0xffffu;
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(q0 * UP, q1 * UP, 0, false) & 0xffffu;
-  if (lo == hi && v0 == v0 && v1 == v1)
-    return mid;
-  const double step0 = a.scales ? 1.0 / a.scales[n0] : a.step, step1 = a.scales ? 1.0 / a.scales[n1] : a.step;
-  return f8_requant_exact(v0, step0) | (f8_requant_exact(v1, step1) << 8);
-}
-
-constexpr int F8_STRIDE = 68;  // dwords per row of an epilogue strip (64 + 4: 16-byte aligned rows, staggered banks)
-
-// Epilogue of a wave's 64 x 64 block through its own strip of LDS: the accumulators (register r of lane l = row
-// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of block (i, j)) are laid out row-major so that a lane owns 16
-// consecutive columns of a row -- per-column parameters are fetched once per lane, results leave as 16-byte stores.
-// WT = edge of the wave's square of outputs (64: 2 x 2 blocks, 32: one block); the strip has WT + 4 dwords per row
-template <int FMT, int WT = 64>
-__device__ __forceinline__ void f8_strip_epilogue(const F8Args &a, const f32x16 (&acc)[WT / 32][WT / 32], float *strip,
-                                                  int64_t m0, int64_t nb, int lane) {
-  constexpr int NB = WT / 32, F8_STRIDE = WT + 4;
-  constexpr int CPR = WT / 16, RPP = 64 / CPR, PASSES = WT / RPP;  // 16-column chunks per row, rows per pass, passes
+  c.n0 = n0;
+  c.whole = n0 + 16 <= a.N;
+  // every load of an array is on its way before the first is used
+  auto at = [&](int e) { return (n0 + e) < a.N ? (n0 + e) : (a.N - 1); };
 #pragma unroll
-  for (int i = 0; i < NB; ++i)
+  for (int e = 0; e < 16; ++e)
+    c.bias[e] = 0.0f;
+  if (a.bias) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
+    for (int e = 0; e < 16; ++e)
+      c.bias[e] = a.bias[at(e)];
+  }
+  float inv[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        strip[(i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * F8_STRIDE + j * 32 + (lane & 31)] = acc[i][j][r];
-  // a wave only reads what it wrote: no barrier, the LDS counter orders it
-  const int cc = lane % CPR, rsub = lane / CPR;  // 16-column chunk, row within a group of RPP rows
-  const int64_t n0 = nb + cc * 16;
-  const bool vec_ok = (a.N % 16) == 0 && n0 + 16 <= a.N;
-  float bias[16], inv[16];  // per column: bias, fl32(1 / step)
+  for (int e = 0; e < 16; ++e)
+    inv[e] = a.inv_step;
+  if (a.scales) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      inv[e] = (float)a.scales[at(e)];
+  }
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
-    const int64_t n = (n0 + e) < a.N ? (n0 + e) : (a.N - 1);
-    bias[e] = a.bias ? a.bias[n] : 0.0f;
-    inv[e] = a.scales ? (float)a.scales[n] : a.inv_step;
+    c.inv_lo[e] = inv[e] * DN;
+    c.inv_hi[e] = inv[e] * UP;
   }
-  const float relu_hi = (a.do_relu && a.relu_limit > 0.0f) ? a.relu_limit : __builtin_inff();
+}
+template <typename V>
+__device__ __forceinline__ void f8_store16(void *p, V v) {
+  static_assert(sizeof(V) == 16, "16 bytes");
+  __builtin_memcpy(p, &v, 16);
+}
+
+// The output kinds and row ends that are not 16 whole codes: n codes as codes or as the values they stand for (exact in
+// all three types).  Out of line: the finishing loop is instantiated several times.
+__device__ __attribute__((noinline)) void f8_store_codes(void *out, int kind, int64_t o, int n, uint32_t w0, uint32_t w1,
+                                                         uint32_t w2, uint32_t w3) {
+  const uint32_t w[4] = {w0, w1, w2, w3};
+  auto code = [&](int e) { return (w[e >> 2] >> (8 * (e & 3))) & 0xffu; };
+  if (kind == MI_F8_OUT_CODES) {
 #pragma unroll
-  for (int p = 0; p < PASSES; ++p) {
-    const int row = p * RPP + rsub;
-    const int64_t m = m0 + row;
-    float v[16];
+    for (int e = 0; e < 16; ++e)
+      if (e < n)
+        ((uint8_t *)out)[o + e] = (uint8_t)code(e);
+    return;
+  }
+  if (kind == MI_F8_OUT_F32) {
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) {
-      const f32x4 t = *(const f32x4 *)(strip + row * F8_STRIDE + cc * 16 + q4 * 4);
-      v[q4 * 4 + 0] = t[0];
-      v[q4 * 4 + 1] = t[1];
-      v[q4 * 4 + 2] = t[2];
-      v[q4 * 4 + 3] = t[3];
-    }
+      float v[4];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      v[e] += bias[e];
-      if (a.do_relu) {  // post_relu, lib/Support/Dnnl/DnnlUtils.cpp:15-25 (its comparison sends a NaN to 0 as well)
-        v[e] = v[e] > 0.0f ? v[e] : 0.0f;
-        v[e] = v[e] > relu_hi ? relu_hi : v[e];
+      for (int e = 0; e < 4; ++e)
+        v[e] = f8e4m3_to_f32(code(q4 * 4 + e));
+      if (q4 * 4 + 4 <= n) {
+        f8_store16((float *)out + o + q4 * 4, f32x4{v[0], v[1], v[2], v[3]});
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (q4 * 4 + e < n)
+            ((float *)out)[o + q4 * 4 + e] = v[e];
       }
     }
-    if (m >= a.M)
-      continue;
-    const int64_t o = m * a.N + n0;
-    if constexpr (FMT == F8_FMT_E5M2) {
-      if (vec_ok && a.acc_out) {
+    return;
+  }
 #pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4)
-          *(f32x4 *)(a.acc_out + o + q4 * 4) = f32x4{v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3]};
-      }
-      if (vec_ok && a.out_kind == MI_F8_OUT_CODES) {
-        uint32_t w[4];
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4)
-          w[q4] = f8e5m2_from_f32(v[q4 * 4]) | (f8e5m2_from_f32(v[q4 * 4 + 1]) << 8) |
-                  (f8e5m2_from_f32(v[q4 * 4 + 2]) << 16) | (f8e5m2_from_f32(v[q4 * 4 + 3]) << 24);
-        *(u32x4 *)((uint8_t *)a.out + o) = u32x4{w[0], w[1], w[2], w[3]};
-        continue;
-      }
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        if (n0 + e >= a.N)
-          continue;
-        if (a.acc_out && !vec_ok)
-          a.acc_out[o + e] = v[e];
-        f8_store_e5m2(a, o + e, v[e]);
-      }
-      continue;
-    }
-    uint32_t c2[8];  // two codes each
+  for (int q8 = 0; q8 < 2; ++q8) {
+    uint32_t h[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const int64_t n_a = (n0 + 2 * e) < a.N ? (n0 + 2 * e) : (a.N - 1);
-      const int64_t n_b = (n0 + 2 * e + 1) < a.N ? (n0 + 2 * e + 1) : (a.N - 1);
-      c2[e] = f8_requant_pair(a, v[2 * e], v[2 * e + 1], inv[2 * e], inv[2 * e + 1], n_a, n_b);
+      const float v = f8e4m3_to_f32(code(q8 * 8 + e));
+      h[e] = kind == MI_F8_OUT_BF16 ? __float_as_uint(v) >> 16 : __builtin_bit_cast(uint16_t, (_Float16)v);
     }
-    if (vec_ok) {
-      if (a.acc_out) {
+    if (q8 * 8 + 8 <= n) {
+      f8_store16((uint16_t *)out + o + q8 * 8,
+                 u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)});
+    } else {
 #pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4)
-          *(f32x4 *)(a.acc_out + o + q4 * 4) = f32x4{v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3]};
-      }
-      if (a.out_kind == MI_F8_OUT_CODES) {
-        *(u32x4 *)((uint8_t *)a.out + o) = u32x4{c2[0] | (c2[1] << 16), c2[2] | (c2[3] << 16), c2[4] | (c2[5] << 16),
-                                                 c2[6] | (c2[7] << 16)};
-        continue;
-      }
+      for (int e = 0; e < 8; ++e)
+        if (q8 * 8 + e < n)
+          ((uint16_t *)out)[o + q8 * 8 + e] = (uint16_t)h[e];
     }
+  }
+}
+
+// One row of a lane's 16 columns, read from the strip: bias, ReLU, side output, requantization, store.
+template <int FMT>
+__device__ __forceinline__ void f8_finish_row(const F8Args &a, const F8Cols &c, const float *src, int64_t m) {
+  float v[16];
+#pragma unroll
+  for (int q4 = 0; q4 < 4; ++q4) {
+    const f32x4 t = *(const f32x4 *)(src + q4 * 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v[q4 * 4 + e] = t[e] + c.bias[q4 * 4 + e];
+  }
+  if (a.do_relu) {  // post_relu, lib/Support/Dnnl/DnnlUtils.cpp:15-25 (its comparison sends a NaN to 0 as well)
+    const float relu_hi = a.relu_limit > 0.0f ? a.relu_limit : __builtin_inff();
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      if (n0 + e >= a.N)
-        continue;
-      if (a.acc_out && !vec_ok)
-        a.acc_out[o + e] = v[e];
-      const uint32_t code = (c2[e >> 1] >> (8 * (e & 1))) & 0xffu;
-      if (a.out_kind == MI_F8_OUT_CODES)
-        ((uint8_t *)a.out)[o + e] = (uint8_t)code;
-      else if (a.out_kind == MI_F8_OUT_F32)
-        ((float *)a.out)[o + e] = f8e4m3_to_f32(code);
-      else if (a.out_kind == MI_F8_OUT_BF16)  // exact: E4M3 values fit both 16-bit types
-        ((uint16_t *)a.out)[o + e] = (uint16_t)(__float_as_uint(f8e4m3_to_f32(code)) >> 16);
-      else
-        ((uint16_t *)a.out)[o + e] = __builtin_bit_cast(uint16_t, (_Float16)f8e4m3_to_f32(code));
+      v[e] = v[e] > 0.0f ? v[e] : 0.0f;
+      v[e] = v[e] > relu_hi ? relu_hi : v[e];
     }
+  }
+  if (m >= a.M || c.n0 >= a.N)
+    return;
+  const int64_t o = m * a.N + c.n0;
+  if (a.acc_out) {
+    if (c.whole) {
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        f8_store16(a.acc_out + o + q4 * 4, f32x4{v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3]});
+    } else {
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (c.n0 + e < a.N)
+          a.acc_out[o + e] = v[e];
+    }
+  }
+  if constexpr (FMT == F8_FMT_E5M2) {
+    if (c.whole && a.out_kind == MI_F8_OUT_CODES) {
+      uint32_t w[4];
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        w[q4] = f8e5m2_from_f32(v[q4 * 4]) | (f8e5m2_from_f32(v[q4 * 4 + 1]) << 8) |
+                (f8e5m2_from_f32(v[q4 * 4 + 2]) << 16) | (f8e5m2_from_f32(v[q4 * 4 + 3]) << 24);
+      f8_store16((uint8_t *)a.out + o, u32x4{w[0], w[1], w[2], w[3]});
+      return;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      if (c.n0 + e < a.N)
+        f8_store_e5m2(a, o + e, v[e]);
+    return;
+  } else {
+    uint32_t w[4];  // four codes each
+    uint32_t differ = 0;
+    bool nan = false;
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      auto clamped = [](float q) { return __builtin_amdgcn_fmed3f(q, -448.0f, 448.0f); };
+      int lo = 0, hi = 0;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int e = q4 * 4 + u * 2;
+        const float l0 = clamped(v[e] * c.inv_lo[e]), l1 = clamped(v[e + 1] * c.inv_lo[e + 1]);
+        const float h0 = clamped(v[e] * c.inv_hi[e]), h1 = clamped(v[e + 1] * c.inv_hi[e + 1]);
+        lo = u ? __builtin_amdgcn_cvt_pk_fp8_f32(l0, l1, lo, true) : __builtin_amdgcn_cvt_pk_fp8_f32(l0, l1, lo, false);
+        hi = u ? __builtin_amdgcn_cvt_pk_fp8_f32(h0, h1, hi, true) : __builtin_amdgcn_cvt_pk_fp8_f32(h0, h1, hi, false);
+        nan |= __builtin_isunordered(v[e], v[e + 1]);
+      }
+      w[q4] = (uint32_t)lo;
+      differ |= (uint32_t)(lo != hi) << q4;
+    }
+    if (differ != 0 || nan) {
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        if (nan || ((differ >> q4) & 1))
+          w[q4] = f8_requant_exact4(v[q4 * 4], v[q4 * 4 + 1], v[q4 * 4 + 2], v[q4 * 4 + 3], a.scales, c.n0 + q4 * 4, a.N - 1,
+                                    a.step);
+    }
+    if (c.whole && a.out_kind == MI_F8_OUT_CODES) {
+      f8_store16((uint8_t *)a.out + o, u32x4{w[0], w[1], w[2], w[3]});
+      return;
+    }
+    const int64_t left = a.N - c.n0;
+    f8_store_codes(a.out, a.out_kind, o, left < 16 ? (int)left : 16, w[0], w[1], w[2], w[3]);
+  }
+}
+
+// Epilogue of NBI x NBJ blocks of a wave through its own strip of LDS: the accumulators (register r of lane l = row
+// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of block (i, j)) are laid out row-major (NBJ * 32 + 4 dwords a row:
+// 16-byte aligned, staggered banks) so that a lane owns 16 consecutive columns of a row -- per-column parameters are
+// fetched once per lane, results leave as 16-byte stores.
+template <int NBJ>
+__device__ __forceinline__ int f8_strip_col(int lane) { return lane % (NBJ * 2) * 16; }
+template <int FMT, int NBI, int NBJ>
+__device__ __forceinline__ void f8_strip_epilogue(const F8Args &a, const f32x16 (&acc)[NBI][NBJ], const F8Cols &cols, float *strip,
+                                                  int64_t m0, int lane) {
+  constexpr int STRIDE = NBJ * 32 + 4, CPR = NBJ * 2, RPP = 64 / CPR, PASSES = NBI * 32 / RPP;
+#pragma unroll
+  for (int i = 0; i < NBI; ++i)
+#pragma unroll
+    for (int j = 0; j < NBJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        strip[(i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * STRIDE + j * 32 + (lane & 31)] = acc[i][j][r];
+  // a wave only reads what it wrote: no barrier, the LDS counter orders it
+#pragma unroll 1
+  for (int p = 0; p < PASSES; ++p) {
+    const int row = p * RPP + lane / CPR;
+    f8_finish_row<FMT>(a, cols, strip + row * STRIDE + f8_strip_col<NBJ>(lane), m0 + row);
   }
 }
 
@@ -465,29 +544,39 @@ __global__ __launch_bounds__(256) void f8_gemm_ring_kernel(F8Args a, int tiles_m
   }
   __builtin_amdgcn_s_waitcnt(f8_waitcnt_vm(0));  // drain the re-loads issued past the end
   __builtin_amdgcn_s_barrier();                  // every wave is done reading the ring
-  f8_strip_epilogue<FMT, WT>(a, acc, (float *)f8_lds + wave * (WT * (WT + 4)), m_base + wm * WT, n_base + wn * WT, lane);
+  F8Cols cols;
+  f8_load_cols(a, cols, n_base + wn * WT + f8_strip_col<NB>(lane));
+  f8_strip_epilogue<FMT, NB, NB>(a, acc, cols, (float *)f8_lds + wave * (WT * (WT + 4)), m_base + wm * WT, lane);
 }
 
-// ---- 256 x 256 outputs per workgroup, 4 waves (2 x 2), each wave 128 x 128 as 4 x 4 blocks of 32 x 32 (256 fp32
-// accumulators per lane).  K advances 64 bytes per stage through a 4-stage LDS ring (32 KiB per stage) filled by
-// direct-to-LDS loads.  One stage = one batch of 16 matrix instructions per wave; the fragment reads of the next stage
-// and the requests of a later one are pinned between them so that they issue in the matrix pipeline's shadow.  One
-// barrier per stage: by then every wave holds the fragments of stage kt in registers (its LDS buffer is free for stage
-// kt + NST) and has received its own share of stage kt + 1.
+// ---- 256 x 256 outputs per workgroup, eight waves (2 x 4, two per SIMD: one wave's waits run under the other's matrix
+// instructions), each 128 x 64 as 4 x 2 blocks of 32 x 32 (128 fp32 accumulators per lane).  K advances 64 bytes per
+// stage, one matrix instruction per block; five stages of 32 KiB fill all of LDS.  As in the INT8 kernel of this tile
+// (i8_kernels.hip) stages are requested in pairs, the two halves of every 128-byte line back to back, so that the vector
+// cache asks L2 for each line once.  Requires K % 128 == 0.  4096^3, per-channel scales: 61.5 us (2.23 PFLOP/s; four
+// waves of 128 x 128 with single-stage requests and the longer epilogue: 84.8); the vendor's fp8 product without
+// requantization reaches 2.77 at this size.
+//
+// A stage is a batch of eight matrix instructions with the next stage's twelve fragment reads and, in every second
+// batch, the eight requests of a pair of stages pinned between them.  The left fragments of the next stage take the
+// registers of this stage's as soon as their two instructions are issued; the right ones alternate between two sets.
+// One barrier per stage, at its start: by then every wave has received the stage's fragments (its LDS buffer is free)
+// and its own share of the next stage, and so after it the next stage is complete.  The pair (2p + 4, 2p + 5) takes
+// the buffers of stages 2p - 1 and 2p, is requested in batch 2p and first read in batch 2p + 3.
 constexpr int F8L_M = 256, F8L_N = 256;
 constexpr int F8L_STAGE = (F8L_M + F8L_N) * F8_BK;  // 32 KiB
-constexpr int F8L_NST = 4;
+constexpr int F8L_NST = 5;
 constexpr int F8_WAITCNT_LGKM0 = 0xC07F;
 
 template <int FMT>
-__global__ __launch_bounds__(256, 1) void f8_gemm_large_kernel(F8Args a, int tiles_m, int tiles_n, int per_xcd) {
+__global__ __launch_bounds__(512, 1) void f8_gemm_large_kernel(F8Args a, int tiles_m, int tiles_n, int per_xcd) {
   constexpr int NST = F8L_NST;
-  constexpr int LOADS = F8L_M * (F8_BK / 16) / 256;  // direct-to-LDS instructions per operand, stage and thread: 4
-  constexpr int LPS = 2 * LOADS;
+  constexpr int LOADS = F8L_M * (F8_BK / 16) / 512;  // direct-to-LDS instructions per operand, stage and thread: 2
+  constexpr int PAIR = 4 * LOADS;                    // requests per thread and pair of stages
   extern __shared__ __attribute__((aligned(16))) uint8_t f8_lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave >> 2, wn = wave & 3;
   const int bid = blockIdx.x;
   const int L = (bid & 7) * per_xcd + (bid >> 3);  // each XCD gets a contiguous run of the tile order
   if (L >= tiles_m * tiles_n)
@@ -499,35 +588,37 @@ __global__ __launch_bounds__(256, 1) void f8_gemm_large_kernel(F8Args a, int til
   const int tm = group * GM + in_group % gm, tn = in_group / gm;
   const int64_t m_base = (int64_t)tm * F8L_M, n_base = (int64_t)tn * F8L_N;
 
-  const uint8_t *ga[LOADS], *gb[LOADS];
+  // a lane's address is a uniform tile base plus a 32-bit offset (rows past the matrix re-read the last one; their
+  // results are never stored); the 16-byte chunk c of row r is stored at position c ^ ((r >> 2) & 3)
+  const uint8_t *Abase = a.A + m_base * a.K, *Bbase = a.B + n_base * a.K;
+  uint32_t va[LOADS], vb[LOADS];
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
-    const int slot = (i * 4 + wave) * 64 + lane;
-    const int row = slot >> 2, pos = slot & 3;
-    const int chunk = pos ^ ((row >> 2) & 3);
+    const int slot = (i * 8 + wave) * 64 + lane;
+    const int row = slot >> 2, chunk = (slot & 3) ^ ((row >> 2) & 3);
     int64_t ra = m_base + row, rb = n_base + row;
-    ra = ra < a.M ? ra : a.M - 1;  // rows past the matrix re-read the last one; their results are never stored
+    ra = ra < a.M ? ra : a.M - 1;
     rb = rb < a.N ? rb : a.N - 1;
-    ga[i] = a.A + ra * a.K + chunk * 16;
-    gb[i] = a.B + rb * a.K + chunk * 16;
+    va[i] = (uint32_t)((ra - m_base) * a.K + chunk * 16);
+    vb[i] = (uint32_t)((rb - n_base) * a.K + chunk * 16);
   }
-  const int kt_total = (int)(a.K / F8_BK);
-  // request q (0 .. LPS-1) of stage kt: even q operand A, odd q operand B
-  auto issue_one = [&](int kt, int q) {
-    const int64_t koff = (int64_t)(kt < kt_total ? kt : kt_total - 1) * F8_BK;  // past the end: harmless re-load
-    uint8_t *sa = f8_lds + (kt % NST) * F8L_STAGE, *sb = sa + F8L_M * F8_BK;
-    const int li = q >> 1;
-    if (q & 1)
-      __builtin_amdgcn_global_load_lds((f8_gptr_t)(gb[li] + koff), (f8_lptr_t)(sb + (li * 4 + wave) * 1024), 16, 0, 0);
-    else
-      __builtin_amdgcn_global_load_lds((f8_gptr_t)(ga[li] + koff), (f8_lptr_t)(sa + (li * 4 + wave) * 1024), 16, 0, 0);
+  const int pairs = (int)(a.K / (2 * F8_BK));
+  // one operand (half = 0: A, 1: B), one of its LOADS pieces of a pair of stages; s0, s1: their buffers
+  auto issue = [&](int pair, int half, int i, int s0, int s1) {
+    const int64_t koff = (int64_t)(pair < pairs ? pair : pairs - 1) * (2 * F8_BK);  // past the end: harmless re-load
+    const uint8_t *pg = (half ? Bbase : Abase) + koff;
+    const uint32_t v = half ? vb[i] : va[i];
+    uint8_t *l0 = f8_lds + s0 * F8L_STAGE + half * (F8L_M * F8_BK) + (i * 8 + wave) * 1024;
+    uint8_t *l1 = f8_lds + s1 * F8L_STAGE + half * (F8L_M * F8_BK) + (i * 8 + wave) * 1024;
+    __builtin_amdgcn_global_load_lds((f8_gptr_t)(pg + v), (f8_lptr_t)l0, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((f8_gptr_t)(pg + v + F8_BK), (f8_lptr_t)l1, 16, 0, 0);
   };
 
-  f32x16 acc[4][4];
+  f32x16 acc[4][2];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         acc[i][j][r] = 0.0f;
@@ -535,81 +626,62 @@ __global__ __launch_bounds__(256, 1) void f8_gemm_large_kernel(F8Args a, int til
   const int frow = lane & 31, kh = lane >> 5;
   const int f_sw = (frow >> 2) & 3;
   const int c0 = (kh ^ f_sw) << 4, c1 = ((2 + kh) ^ f_sw) << 4;  // this lane's two chunks of a row, swizzled
-  int a_off[4], b_off[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    a_off[i] = (wm * 128 + i * 32 + frow) * F8_BK;
-    b_off[i] = F8L_M * F8_BK + (wn * 128 + i * 32 + frow) * F8_BK;
-  }
+  const int a_row = (wm * 128 + frow) * F8_BK, b_row = F8L_M * F8_BK + (wn * 64 + frow) * F8_BK;
   auto read_frag = [&](i32x8 &f, const uint8_t *st, int off) {
     const u32x4 lo = *(const u32x4 *)(st + off + c0), hi = *(const u32x4 *)(st + off + c1);
     f = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
   };
 
-  // one stage: wait, barrier, then 16 matrix instructions on the fragments of stage kt with the 8 fragment reads of
-  // stage kt + 1 and the 8 requests of stage kt + NST pinned between them
-  auto stage = [&](const i32x8 (&ca)[4], const i32x8 (&cb)[4], i32x8 (&na)[4], i32x8 (&nb)[4], int kt) {
-    __builtin_amdgcn_s_waitcnt(F8_WAITCNT_LGKM0);                // the fragments of stage kt are in registers
-    __builtin_amdgcn_s_waitcnt(f8_waitcnt_vm((NST - 2) * LPS));  // this thread's share of stage kt + 1 has landed
+  i32x8 fa[4], fb[2][2];
+  // batch kt: its fragments are in fa and fb[cur]; pair >= 0: that pair of stages is requested on the way
+  auto batch = [&](int cur, int kt, int pair) {
+    __builtin_amdgcn_s_waitcnt(F8_WAITCNT_LGKM0);
+    __builtin_amdgcn_s_waitcnt(f8_waitcnt_vm(PAIR));  // all but the newest pair of stages
     __builtin_amdgcn_s_barrier();
-    const uint8_t *st = f8_lds + ((kt + 1) % NST) * F8L_STAGE;
+    const uint8_t *st = f8_lds + (kt + 1) % NST * F8L_STAGE;
+    const int s0 = (kt + 4) % NST, s1 = kt % NST;  // pair: the buffers of stages kt + 4 and kt + 5
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const int i = t >> 2, j = t & 3;
-      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ca[i], cb[j], acc[i][j], FMT, FMT, 0, 0, 0, 0);
-      if (t < 4)
-        read_frag(na[t], st, a_off[t]);
-      else if (t < 8)
-        read_frag(nb[t - 4], st, b_off[t - 4]);
-      else
-        issue_one(kt + NST, t - 8);
+    for (int t = 0; t < 8; ++t) {
+      const int i = t >> 1, j = t & 1;
+      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa[i], fb[cur][j], acc[i][j], FMT, FMT, 0, 0, 0, 0);
+      if (j)
+        read_frag(fa[i], st, a_row + i * 32 * F8_BK);
+      else if (i < 2)
+        read_frag(fb[cur ^ 1][i], st, b_row + i * 32 * F8_BK);
+      if (pair >= 0 && t >= 4)
+        issue(pair, (t - 4) >> 1, (t - 4) & 1, s0, s1);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-
 #pragma unroll
-  for (int s0 = 0; s0 < NST; ++s0)
+  for (int p = 0; p < 2; ++p)
 #pragma unroll
-    for (int q = 0; q < LPS; ++q)
-      issue_one(s0, q);
-  i32x8 fa[2][4], fb[2][4];
-  __builtin_amdgcn_s_waitcnt(f8_waitcnt_vm((NST - 1) * LPS));  // stage 0 landed
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i)
+        issue(p, half, i, 2 * p, 2 * p + 1);
+  __builtin_amdgcn_s_waitcnt(f8_waitcnt_vm(PAIR));  // stages 0 and 1 landed
   __builtin_amdgcn_s_barrier();
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    read_frag(fa[0][i], f8_lds, a_off[i]);
-    read_frag(fb[0][i], f8_lds, b_off[i]);
+  for (int i = 0; i < 4; ++i)
+    read_frag(fa[i], f8_lds, a_row + i * 32 * F8_BK);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    read_frag(fb[0][j], f8_lds, b_row + j * 32 * F8_BK);
+  for (int p = 0; p < pairs; ++p) {
+    batch(0, 2 * p, p + 2);
+    batch(1, 2 * p + 1, -1);
   }
-  int kt = 0;
-  for (; kt + 1 < kt_total; kt += 2) {
-    stage(fa[0], fb[0], fa[1], fb[1], kt);
-    stage(fa[1], fb[1], fa[0], fb[0], kt + 1);
-  }
-  if (kt < kt_total)
-    stage(fa[0], fb[0], fa[1], fb[1], kt);
   __builtin_amdgcn_s_waitcnt(f8_waitcnt_vm(0));  // drain the re-loads issued past the end
-  __builtin_amdgcn_s_waitcnt(F8_WAITCNT_LGKM0);
-  __builtin_amdgcn_s_barrier();                  // every wave is done with the ring
+  __syncthreads();                               // every wave is done with the ring
 
-  // four 64 x 64 quadrants, written out one by one: inside a loop the accumulator indices would stop being
-  // compile-time constants and the accumulators would move to scratch memory
-  float *strip = (float *)f8_lds + wave * (64 * F8_STRIDE);
-  const int64_t mw = m_base + wm * 128, nw = n_base + wn * 128;
-  {
-    const f32x16 sub[2][2] = {{acc[0][0], acc[0][1]}, {acc[1][0], acc[1][1]}};
-    f8_strip_epilogue<FMT>(a, sub, strip, mw, nw, lane);
-  }
-  {
-    const f32x16 sub[2][2] = {{acc[0][2], acc[0][3]}, {acc[1][2], acc[1][3]}};
-    f8_strip_epilogue<FMT>(a, sub, strip, mw, nw + 64, lane);
-  }
-  {
-    const f32x16 sub[2][2] = {{acc[2][0], acc[2][1]}, {acc[3][0], acc[3][1]}};
-    f8_strip_epilogue<FMT>(a, sub, strip, mw + 64, nw, lane);
-  }
-  {
-    const f32x16 sub[2][2] = {{acc[2][2], acc[2][3]}, {acc[3][2], acc[3][3]}};
-    f8_strip_epilogue<FMT>(a, sub, strip, mw + 64, nw + 64, lane);
+  F8Cols cols;
+  f8_load_cols(a, cols, n_base + wn * 64 + f8_strip_col<2>(lane));
+  float *strip = (float *)f8_lds + wave * (32 * 68);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x16 sub[1][2] = {{acc[i][0], acc[i][1]}};
+    f8_strip_epilogue<FMT, 1, 2>(a, sub, cols, strip, m_base + wm * 128 + i * 32, lane);
   }
 }
 
@@ -849,7 +921,7 @@ int f8mm_launch(const uint8_t *d_a, const uint8_t *d_b, int right_transpose, con
     lim4b.ensure((const void *)f8_gemm_ring_kernel<4, F8_FMT_E5M2>, f8_ring_lds_bytes(4));
     const int64_t tl_m = (M + F8L_M - 1) / F8L_M, tl_n = (N + F8L_N - 1) / F8L_N;
     const int e = plan().f8_tile;
-    const bool large = e ? e == 256 : tl_m * tl_n >= 144;  // the INT8 kernels' measured crossover
+    const bool large = (K % 128) == 0 && (e ? e == 256 : tl_m * tl_n >= 144);  // the INT8 kernels' measured crossover
     const bool small = e ? e == 64 : tiles <= 128;         // likewise
     if (small && !large) {
       const int64_t ts_m = (M + 63) / 64, ts_n = (N + 63) / 64;
@@ -868,9 +940,9 @@ int f8mm_launch(const uint8_t *d_a, const uint8_t *d_b, int right_transpose, con
       const int tl = (int)(tl_m * tl_n), pl = (tl + 7) / 8;
       const dim3 grid((unsigned)(pl * 8));
       if (e5m2)
-        f8_gemm_large_kernel<F8_FMT_E5M2><<<grid, dim3(256), F8L_NST * F8L_STAGE, stream>>>(a, (int)tl_m, (int)tl_n, pl);
+        f8_gemm_large_kernel<F8_FMT_E5M2><<<grid, dim3(512), F8L_NST * F8L_STAGE, stream>>>(a, (int)tl_m, (int)tl_n, pl);
       else
-        f8_gemm_large_kernel<F8_FMT_E4M3><<<grid, dim3(256), F8L_NST * F8L_STAGE, stream>>>(a, (int)tl_m, (int)tl_n, pl);
+        f8_gemm_large_kernel<F8_FMT_E4M3><<<grid, dim3(512), F8L_NST * F8L_STAGE, stream>>>(a, (int)tl_m, (int)tl_n, pl);
     } else {
       const dim3 grid((unsigned)(per_xcd * 8));
       const int tm = (int)tiles_m, tn = (int)tiles_n;
