@@ -329,3 +329,12 @@ def test_f8_matmul_with_few_rows(orc, plan, M, K, N, rt, relu, per_channel, bias
                                                 (32, 8192, 64, True, False, True)])
 def test_e5m2_matmul_with_few_rows(orc, plan, M, K, N, rt, relu, bias):
     test_e5m2_matmul_device_level(orc, plan, M, K, N, rt, relu, bias, "32")
+
+
+@pytest.mark.parametrize("tile", ["64", "128", "256"])
+@pytest.mark.parametrize("M,K,N,rt", [(1, 1, 1, True), (65, 63, 131, False), (129, 65, 33, True), (130, 127, 259, False),
+                                      (257, 192, 129, True), (40, 1000, 300, False)])
+def test_f8_matmul_rewritten_operands(orc, plan, M, K, N, rt, tile):
+    """K that is no whole number of stages (padded) and [K, N] right operands (transposed), rows at every alignment, in
+    each tile kernel; checks and bounds of test_f8_matmul_device_level."""
+    test_f8_matmul_device_level(orc, plan, M, K, N, rt, M % 2 == 0, K > 64, True, tile)

@@ -7,10 +7,12 @@
 // 128 x 128 outputs per workgroup, 4 waves (2 x 2), each wave 64 x 64 as 2 x 2 blocks of 32 x 32.  K advances 64 bytes per
 // stage; one matrix instruction consumes a whole stage of a block (64 k: lane l holds two 16-byte pieces of row l % 32
 // for both operands -- the contraction order inside an instruction is free as long as both sides agree).
-//   f8_gemm_ring_kernel   K % 64 == 0: a ring of LDS stages filled by direct-to-LDS loads (no staging registers, several
-//                         stages of requests in flight), 16-byte chunks XOR-swizzled against bank conflicts, workgroups
-//                         renumbered so that each XCD's L2 sees a compact block of tiles.
-//   f8_gemm_kernel        any K: operands staged through registers into two padded LDS stages.
+//   f8_gemm_ring_kernel   a ring of LDS stages filled by direct-to-LDS loads (no staging registers, several stages of
+//                         requests in flight), 16-byte chunks XOR-swizzled against bank conflicts, workgroups renumbered
+//                         so that each XCD's L2 sees a compact block of tiles.
+//   f8_gemm_large_kernel  the same for 256 x 256 tiles.
+// A [K, N] right operand, and a K that is no whole number of stages, is rewritten first (operand_copy.hip; code 0 = +0:
+// padding adds nothing).
 //
 // The fp8 matrix pipeline aligns the products of one instruction to the largest and drops low bits, so a long sum
 // carries a relative error of about 2^-13 where an fp32 FMA chain has 2^-24; after the E4M3 rounding (2^-4 steps) that
@@ -29,7 +31,6 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 constexpr int F8_BM = 128, F8_BN = 128, F8_BK = 64;
-constexpr int F8_LDS_ROW = 80;
 
 struct F8Args {
   const uint8_t *A;     // [M, K] E4M3 codes
@@ -50,27 +51,6 @@ struct F8Args {
   unsigned *counters;   // [block], zero between launches
 };
 
-__device__ __forceinline__ u32x4 f8_load_chunk(const uint8_t *base, int64_t row, int64_t rows, int64_t k, int64_t K,
-                                               bool vec_ok) {
-  u32x4 v = {0, 0, 0, 0};  // code 0 = +0: rows and columns past the matrix add nothing
-  if (row < rows && k < K) {
-    const uint8_t *p = base + row * K + k;
-    if (vec_ok && k + 16 <= K) {
-      v = *(const u32x4 *)p;
-    } else {
-      uint8_t tmp[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        tmp[i] = (k + i < K) ? p[i] : (uint8_t)0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[i] = (uint32_t)tmp[4 * i] | ((uint32_t)tmp[4 * i + 1] << 8) | ((uint32_t)tmp[4 * i + 2] << 16) |
-               ((uint32_t)tmp[4 * i + 3] << 24);
-    }
-  }
-  return v;
-}
-
 // operand format of v_mfma_f32_32x32x64_f8f6f4 (its cbsz / blgp fields): 0 = E4M3, 1 = E5M2
 constexpr int F8_FMT_E4M3 = 0, F8_FMT_E5M2 = 1;
 
@@ -87,80 +67,6 @@ __device__ __forceinline__ void f8_store_e5m2(const F8Args &a, int64_t o, float 
     ((uint16_t *)a.out)[o] = f32_to_f16_ref(v);
 }
 
-template <int FMT>
-__device__ __forceinline__ void f8_epilogue(const F8Args &a, const f32x16 (&acc)[2][2], int64_t m0, int64_t n0, int lane);
-
-template <int FMT>
-__global__ __launch_bounds__(256) void f8_gemm_kernel(F8Args a) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds_a[2][F8_BM * F8_LDS_ROW];
-  __shared__ __attribute__((aligned(16))) uint8_t lds_b[2][F8_BN * F8_LDS_ROW];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int64_t m_base = (int64_t)blockIdx.y * F8_BM, n_base = (int64_t)blockIdx.x * F8_BN;
-  const bool vec_ok = (a.K % 16) == 0;
-
-  // staging: 128 rows x 4 chunks of 16 B per operand tile = 512 chunks, two per thread
-  const int c_row0 = tid >> 2, c_col = tid & 3;  // rows c_row0 and c_row0 + 64
-  u32x4 ra[2], rb[2];
-  auto gload = [&](int64_t k0) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      ra[h] = f8_load_chunk(a.A, m_base + c_row0 + 64 * h, a.M, k0 + 16 * c_col, a.K, vec_ok);
-      rb[h] = f8_load_chunk(a.B, n_base + c_row0 + 64 * h, a.N, k0 + 16 * c_col, a.K, vec_ok);
-    }
-  };
-  auto lstore = [&](int stage) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      *(u32x4 *)&lds_a[stage][(c_row0 + 64 * h) * F8_LDS_ROW + 16 * c_col] = ra[h];
-      *(u32x4 *)&lds_b[stage][(c_row0 + 64 * h) * F8_LDS_ROW + 16 * c_col] = rb[h];
-    }
-  };
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        acc[i][j][r] = 0.0f;
-
-  const int64_t k_iters = (a.K + F8_BK - 1) / F8_BK;
-  gload(0);
-  lstore(0);
-  __syncthreads();
-  const int frow = lane & 31, fk = (lane >> 5) * 32;
-  for (int64_t it = 0; it < k_iters; ++it) {
-    const int stage = (int)(it & 1);
-    if (it + 1 < k_iters)
-      gload((it + 1) * F8_BK);
-    i32x8 fa[2], fb[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const uint8_t *pa = &lds_a[stage][(wm * 64 + i * 32 + frow) * F8_LDS_ROW + fk];
-      const uint8_t *pb = &lds_b[stage][(wn * 64 + i * 32 + frow) * F8_LDS_ROW + fk];
-      const u32x4 a0 = *(const u32x4 *)pa, a1 = *(const u32x4 *)(pa + 16);
-      const u32x4 b0 = *(const u32x4 *)pb, b1 = *(const u32x4 *)(pb + 16);
-      fa[i] = i32x8{(int)a0[0], (int)a0[1], (int)a0[2], (int)a0[3], (int)a1[0], (int)a1[1], (int)a1[2], (int)a1[3]};
-      fb[i] = i32x8{(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3], (int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)  // formats 0 / 0 = E4M3 x E4M3, no block scales
-        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa[i], fb[j], acc[i][j], FMT, FMT, 0, 0, 0, 0);
-    if (it + 1 < k_iters) {
-      lstore(stage ^ 1);
-      __syncthreads();
-    }
-  }
-
-  f8_epilogue<FMT>(a, acc, m_base + wm * 64, n_base + wn * 64, lane);
-}
-
-// epilogue of a wave's 64 x 64 block: register r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of its
-// 32 x 32 block (i, j)
 // One output: bias added by the caller; ReLU, the fp32 side output, the requantization and the store.
 template <int FMT>
 __device__ __forceinline__ void f8_finish_one(const F8Args &a, int64_t o, float v, double step, double inv_step) {
@@ -191,27 +97,6 @@ __device__ __forceinline__ void f8_finish_one(const F8Args &a, int64_t o, float 
     ((uint16_t *)a.out)[o] = (uint16_t)(__float_as_uint(f8e4m3_to_f32(code)) >> 16);
   else
     ((uint16_t *)a.out)[o] = __builtin_bit_cast(uint16_t, (_Float16)f8e4m3_to_f32(code));
-}
-
-template <int FMT>
-__device__ __forceinline__ void f8_epilogue(const F8Args &a, const f32x16 (&acc)[2][2], int64_t m0, int64_t n0, int lane) {
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int64_t n = n0 + j * 32 + (lane & 31);
-    const bool n_ok = n < a.N;
-    const float bias_n = (a.bias && n_ok) ? a.bias[n] : 0.0f;
-    const double step = (a.scales && n_ok) ? 1.0 / a.scales[n] : a.step;
-    const double inv_step = 1.0 / step;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t m = m0 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (n_ok && m < a.M)
-          f8_finish_one<FMT>(a, m * a.N + n, acc[i][j][r] + bias_n, step, inv_step);
-      }
-    }
-  }
 }
 
 // The reference's requantization is E4M3((float)((double)v / step)), Float8.cpp:259-261.  With inv an fp32 number within
@@ -824,20 +709,6 @@ __global__ __launch_bounds__(512) void f8_rows32_kernel(F8Args a) {
   }
 }
 
-__global__ void f8_transpose_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int64_t K, int64_t N) {
-  // [K, N] -> [N, K], 32 x 32 tiles through LDS
-  __shared__ uint8_t tile[32][33];
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-  const int64_t n0 = (int64_t)blockIdx.x * 32, k0 = (int64_t)blockIdx.y * 32;
-  for (int i = ty; i < 32; i += 8)
-    if (k0 + i < K && n0 + tx < N)
-      tile[i][tx] = src[(k0 + i) * N + n0 + tx];
-  __syncthreads();
-  for (int i = ty; i < 32; i += 8)
-    if (n0 + i < N && k0 + tx < K)
-      dst[(n0 + i) * K + k0 + tx] = tile[tx][i];
-}
-
 int f8mm_launch(const uint8_t *d_a, const uint8_t *d_b, int right_transpose, const float *d_bias, int64_t M, int64_t K,
                 int64_t N, int do_relu, double relu_limit, double out_scale, const double *d_out_scales, int out_kind,
                 void *d_out, float *d_acc, hipStream_t stream, int f8_type) {
@@ -851,26 +722,46 @@ int f8mm_launch(const uint8_t *d_a, const uint8_t *d_b, int right_transpose, con
   MI_REQUIRE(out_kind >= MI_F8_OUT_CODES && out_kind <= MI_F8_OUT_F16, MI_BAD_ARGUMENT, "mi_f8mm_launch: out_kind");
   MI_REQUIRE(d_out_scales || (out_scale == out_scale && out_scale != 0.0), MI_BAD_ARGUMENT,
              "mi_f8mm_launch: the output scale must be a nonzero number");
-  MI_REQUIRE((M + F8_BM - 1) / F8_BM <= 65535, MI_UNSUPPORTED, "mi_f8mm_launch: M too large for one launch");
   if (M == 0)
     return MI_SUCCESS;
-  const uint8_t *b_nk = d_b;
-  if (!right_transpose) {  // [K, N] -> [N, K] into the stream's scratch buffer
-    uint8_t *t = nullptr;
-    int rc = stream_workspace(stream, WS_F8_TRANSPOSE, (size_t)N * K, (void **)&t);
+  // kernel by size: the streaming kernel up to 32 rows, by the INT8 product's rule (same bytes per element; plan: f8_tile
+  // = 32 asks for it, any other value rules it out; 4096 x 4096 (N x K) M = 1: 15.2 us on 64 x 64 tiles, 4096 x 11008:
+  // 38.7), 256 x 256 tiles from the INT8 kernels' measured crossover on, 64 x 64 tiles up to 128 tiles of 128 x 128
+  const int e = plan().f8_tile;
+  const bool few_pays = M * N <= 45056 || (N <= 8192 && (M <= 24 || K > 4096));
+  const bool few = M <= 32 && (K % 128) == 0 && (e == 32 || (e == 0 && few_pays));
+  const int64_t tiles_m = (M + F8_BM - 1) / F8_BM, tiles_n = (N + F8_BN - 1) / F8_BN;
+  const int64_t tl_m = (M + F8L_M - 1) / F8L_M, tl_n = (N + F8L_N - 1) / F8L_N;
+  MI_REQUIRE(tiles_m * tiles_n < (int64_t(1) << 28), MI_UNSUPPORTED, "mi_f8mm_launch: too many outputs for one launch");
+  const bool large = !few && (e > 0 && e != 32 ? e == 256 : tl_m * tl_n >= 144);
+  const bool small = !few && !large && (e > 0 && e != 32 ? e == 64 : tiles_m * tiles_n <= 128);
+  const int64_t stage = large ? 2 * F8_BK : F8_BK, Kp = few ? K : (K + stage - 1) / stage * stage;
+  const bool rewrite_a = Kp != K, rewrite_b = Kp != K || !right_transpose;
+  ScratchBytes scratch;
+  const uint8_t *a_mk = d_a, *b_nk = d_b;
+  if (rewrite_b) {
+    const size_t a_bytes = rewrite_a ? (size_t)((M * Kp + 255) & ~(int64_t)255) : 0;
+    int rc = scratch.get(stream, WS_F8_OPERANDS, a_bytes + (size_t)(N * Kp));
     if (rc != MI_SUCCESS)
       return rc;
-    f8_transpose_kernel<<<dim3((unsigned)((N + 31) / 32), (unsigned)((K + 31) / 32)), dim3(256), 0, stream>>>(d_b, t, K, N);
-    b_nk = t;
+    uint8_t *t = (uint8_t *)scratch.ptr;
+    OperandCopy ca = {}, cb = {d_b, t + a_bytes, N, K, Kp, !right_transpose, 0, 0};
+    if (rewrite_a) {
+      ca = OperandCopy{d_a, t, M, K, Kp, 0, 0, 0};
+      a_mk = t;
+    }
+    b_nk = t + a_bytes;
+    if ((rc = operand_copy_launch(ca, cb, stream)))
+      return rc;
   }
   F8Args a;
-  a.A = d_a;
+  a.A = a_mk;
   a.B = b_nk;
   a.bias = d_bias;
   a.out = d_out;
   a.acc_out = d_acc;
   a.M = M;
-  a.K = K;
+  a.K = Kp;
   a.N = N;
   a.do_relu = do_relu;
   a.relu_limit = (float)relu_limit;
@@ -882,91 +773,62 @@ int f8mm_launch(const uint8_t *d_a, const uint8_t *d_b, int right_transpose, con
   a.part = nullptr;
   a.counters = nullptr;
   const bool e5m2 = f8_type == MI_F8_E5M2;
-  {  // up to 32 rows: the streaming kernel, by the INT8 product's rule (same bytes per element; plan: f8_tile = 32
-     // asks for it, any other value rules it out).  4096 x 4096 (N x K) M = 1: 15.2 us on 64 x 64 tiles, 4096 x 11008: 38.7
-    const bool few_pays = M * N <= 45056 || (N <= 8192 && (M <= 24 || K > 4096));
-    if (M <= 32 && (K % 128) == 0 && (plan().f8_tile == 32 || (plan().f8_tile == 0 && few_pays))) {
-      const int64_t blocks = (N + 31) / 32;
-      MI_REQUIRE(blocks < (1ll << 29), MI_BAD_ARGUMENT, "mi_f8mm_launch: too many output columns");
-      while (a.split_shift < 2 && (blocks << (a.split_shift + 1)) <= R32_SPLIT_MAX_WGS &&
-             K / 128 >= (32 << (a.split_shift + 1)))
-        ++a.split_shift;
-      if (a.split_shift != 0) {
-        void *p = nullptr;
-        // (a stream under capture that never ran such a shape gets the error: an unsplit launch would add the partial
-        // sums in another order)
-        const int rc = stream_workspace(stream, WS_ROWS32_SPLIT, R32_SPLIT_COUNTER_BYTES + (size_t)R32_SPLIT_MAX_WGS * 4096,
-                                        &p, /*zero_fresh=*/true);
-        if (rc != MI_SUCCESS)
-          return rc;
-        a.counters = (unsigned *)p;
-        a.part = (float *)((uint8_t *)p + R32_SPLIT_COUNTER_BYTES);
-      }
-      const dim3 grid((unsigned)(blocks << a.split_shift));
-      if (e5m2)
-        f8_rows32_kernel<F8_FMT_E5M2><<<grid, dim3(512), 0, stream>>>(a);
-      else
-        f8_rows32_kernel<F8_FMT_E4M3><<<grid, dim3(512), 0, stream>>>(a);
-      MI_HIP(hipGetLastError());
-      return MI_SUCCESS;
+  if (few) {
+    const int64_t blocks = (N + 31) / 32;
+    MI_REQUIRE(blocks < (1ll << 29), MI_BAD_ARGUMENT, "mi_f8mm_launch: too many output columns");
+    while (a.split_shift < 2 && (blocks << (a.split_shift + 1)) <= R32_SPLIT_MAX_WGS &&
+           K / 128 >= (32 << (a.split_shift + 1)))
+      ++a.split_shift;
+    if (a.split_shift != 0) {
+      void *p = nullptr;
+      // (a stream under capture that never ran such a shape gets the error: an unsplit launch would add the partial
+      // sums in another order)
+      const int rc = stream_workspace(stream, WS_ROWS32_SPLIT, R32_SPLIT_COUNTER_BYTES + (size_t)R32_SPLIT_MAX_WGS * 4096,
+                                      &p, /*zero_fresh=*/true);
+      if (rc != MI_SUCCESS)
+        return rc;
+      a.counters = (unsigned *)p;
+      a.part = (float *)((uint8_t *)p + R32_SPLIT_COUNTER_BYTES);
     }
-  }
-  const int64_t tiles_m = (M + F8_BM - 1) / F8_BM, tiles_n = (N + F8_BN - 1) / F8_BN;
-  if ((K % F8_BK) == 0 && tiles_m * tiles_n < (int64_t(1) << 30)) {
-    const int tiles = (int)(tiles_m * tiles_n), per_xcd = (tiles + 7) / 8;
-    static LdsLimitOnce lim8a, lim4a, lim8b, lim4b;
-    lim8a.ensure((const void *)f8_gemm_ring_kernel<8, F8_FMT_E4M3>, f8_ring_lds_bytes(8));
-    lim4a.ensure((const void *)f8_gemm_ring_kernel<4, F8_FMT_E4M3>, f8_ring_lds_bytes(4));
-    lim8b.ensure((const void *)f8_gemm_ring_kernel<8, F8_FMT_E5M2>, f8_ring_lds_bytes(8));
-    lim4b.ensure((const void *)f8_gemm_ring_kernel<4, F8_FMT_E5M2>, f8_ring_lds_bytes(4));
-    const int64_t tl_m = (M + F8L_M - 1) / F8L_M, tl_n = (N + F8L_N - 1) / F8L_N;
-    const int e = plan().f8_tile;
-    const bool large = (K % 128) == 0 && (e ? e == 256 : tl_m * tl_n >= 144);  // the INT8 kernels' measured crossover
-    const bool small = e ? e == 64 : tiles <= 128;         // likewise
-    if (small && !large) {
-      const int64_t ts_m = (M + 63) / 64, ts_n = (N + 63) / 64;
-      const int ts = (int)(ts_m * ts_n), ps = (ts + 7) / 8;
-      const dim3 grid((unsigned)(ps * 8));
-      if (e5m2)
-        f8_gemm_ring_kernel<4, F8_FMT_E5M2, 64><<<grid, dim3(256), f8_ring_lds_bytes(4, 64), stream>>>(a, (int)ts_m,
-                                                                                                      (int)ts_n, ps);
-      else
-        f8_gemm_ring_kernel<4, F8_FMT_E4M3, 64><<<grid, dim3(256), f8_ring_lds_bytes(4, 64), stream>>>(a, (int)ts_m,
-                                                                                                      (int)ts_n, ps);
-    } else if (large) {
-      static LdsLimitOnce lim_a, lim_b;
-      lim_a.ensure((const void *)f8_gemm_large_kernel<F8_FMT_E4M3>, F8L_NST * F8L_STAGE);
-      lim_b.ensure((const void *)f8_gemm_large_kernel<F8_FMT_E5M2>, F8L_NST * F8L_STAGE);
-      const int tl = (int)(tl_m * tl_n), pl = (tl + 7) / 8;
-      const dim3 grid((unsigned)(pl * 8));
-      if (e5m2)
-        f8_gemm_large_kernel<F8_FMT_E5M2><<<grid, dim3(512), F8L_NST * F8L_STAGE, stream>>>(a, (int)tl_m, (int)tl_n, pl);
-      else
-        f8_gemm_large_kernel<F8_FMT_E4M3><<<grid, dim3(512), F8L_NST * F8L_STAGE, stream>>>(a, (int)tl_m, (int)tl_n, pl);
-    } else {
-      const dim3 grid((unsigned)(per_xcd * 8));
-      const int tm = (int)tiles_m, tn = (int)tiles_n;
-      if (tiles <= 256) {
-        if (e5m2)
-          f8_gemm_ring_kernel<8, F8_FMT_E5M2><<<grid, dim3(256), f8_ring_lds_bytes(8), stream>>>(a, tm, tn, per_xcd);
-        else
-          f8_gemm_ring_kernel<8, F8_FMT_E4M3><<<grid, dim3(256), f8_ring_lds_bytes(8), stream>>>(a, tm, tn, per_xcd);
-      } else {
-        if (e5m2)
-          f8_gemm_ring_kernel<4, F8_FMT_E5M2><<<grid, dim3(256), f8_ring_lds_bytes(4), stream>>>(a, tm, tn, per_xcd);
-        else
-          f8_gemm_ring_kernel<4, F8_FMT_E4M3><<<grid, dim3(256), f8_ring_lds_bytes(4), stream>>>(a, tm, tn, per_xcd);
-      }
-    }
-  } else {
-    dim3 grid((unsigned)tiles_n, (unsigned)tiles_m);
+    const dim3 grid((unsigned)(blocks << a.split_shift));
     if (e5m2)
-      f8_gemm_kernel<F8_FMT_E5M2><<<grid, dim3(256), 0, stream>>>(a);
+      f8_rows32_kernel<F8_FMT_E5M2><<<grid, dim3(512), 0, stream>>>(a);
     else
-      f8_gemm_kernel<F8_FMT_E4M3><<<grid, dim3(256), 0, stream>>>(a);
+      f8_rows32_kernel<F8_FMT_E4M3><<<grid, dim3(512), 0, stream>>>(a);
+  } else if (large) {
+    static LdsLimitOnce lim_a, lim_b;
+    lim_a.ensure((const void *)f8_gemm_large_kernel<F8_FMT_E4M3>, F8L_NST * F8L_STAGE);
+    lim_b.ensure((const void *)f8_gemm_large_kernel<F8_FMT_E5M2>, F8L_NST * F8L_STAGE);
+    const int per_xcd = (int)((tl_m * tl_n + 7) / 8);
+    const dim3 grid((unsigned)(per_xcd * 8));
+    if (e5m2)
+      f8_gemm_large_kernel<F8_FMT_E5M2><<<grid, dim3(512), F8L_NST * F8L_STAGE, stream>>>(a, (int)tl_m, (int)tl_n, per_xcd);
+    else
+      f8_gemm_large_kernel<F8_FMT_E4M3><<<grid, dim3(512), F8L_NST * F8L_STAGE, stream>>>(a, (int)tl_m, (int)tl_n, per_xcd);
+  } else {
+    const int bt = small ? 64 : 128;
+    const int tm = (int)((M + bt - 1) / bt), tn = (int)((N + bt - 1) / bt), per_xcd = (tm * tn + 7) / 8;
+    const dim3 grid((unsigned)(per_xcd * 8));
+#define MI_F8_RING(NST, BT)                                                                                             \
+  {                                                                                                                     \
+    static LdsLimitOnce lim_a, lim_b;                                                                                   \
+    lim_a.ensure((const void *)f8_gemm_ring_kernel<NST, F8_FMT_E4M3, BT>, f8_ring_lds_bytes(NST, BT));                  \
+    lim_b.ensure((const void *)f8_gemm_ring_kernel<NST, F8_FMT_E5M2, BT>, f8_ring_lds_bytes(NST, BT));                  \
+    if (e5m2)                                                                                                           \
+      f8_gemm_ring_kernel<NST, F8_FMT_E5M2, BT><<<grid, dim3(256), f8_ring_lds_bytes(NST, BT), stream>>>(a, tm, tn, per_xcd); \
+    else                                                                                                                \
+      f8_gemm_ring_kernel<NST, F8_FMT_E4M3, BT><<<grid, dim3(256), f8_ring_lds_bytes(NST, BT), stream>>>(a, tm, tn, per_xcd); \
+  }
+    if (small)
+      MI_F8_RING(4, 64)
+    else if (tiles_m * tiles_n <= 256)
+      MI_F8_RING(8, 128)
+    else
+      MI_F8_RING(4, 128)
+#undef MI_F8_RING
   }
   MI_HIP(hipGetLastError());
-  return MI_SUCCESS;
+  return scratch.release();
 }
 
 }  // namespace mi

@@ -172,7 +172,7 @@ int a16_launch_group(const mi_a16_weight *const *ws, int n, const uint16_t *d_x,
 
 // library-owned scratch, one buffer per (device, stream, purpose) (workspace.hip); contents are whatever the last
 // user left
-enum { WS_SPLIT_K = 0, WS_DYNAMIC_QUANT = 1, WS_F8_TRANSPOSE = 2, WS_ROWS32_SPLIT = 3, WS_I8_OPERANDS = 4 };
+enum { WS_SPLIT_K = 0, WS_DYNAMIC_QUANT = 1, WS_F8_OPERANDS = 2, WS_ROWS32_SPLIT = 3, WS_I8_OPERANDS = 4 };
 // WS_ROWS32_SPLIT, shared by the few-row kernels that split K over workgroups (A16 and INT8): arrival counters, then
 // one 32 x 32 block of partial sums per workgroup.  Always asked for at this one size, so it is never re-allocated.
 constexpr int R32_SPLIT_MAX_WGS = 256;          // workgroups of a split launch, at most
@@ -193,6 +193,16 @@ struct ScratchBytes {
   int get(hipStream_t st, int purpose, size_t bytes);
   int release();  // after the last launch that uses it
 };
+// 8-bit matmul operands in the layout of the tile kernels, both in one launch (operand_copy.hip); src null: none
+struct OperandCopy {
+  const uint8_t *src;
+  uint8_t *dst;        // [rows][Kp], Kp a multiple of 64
+  int64_t rows, K, Kp;
+  int transpose;       // src is [K][rows], else [rows][K]; the second operand only
+  uint32_t flip4;      // XORed into every dword
+  uint32_t pad4;       // what k >= K holds (one byte, four times)
+};
+int operand_copy_launch(const OperandCopy &a, const OperandCopy &b, hipStream_t stream);
 // frees every buffer of a stream (current and retired); for owners of private streams, right before hipStreamDestroy
 void release_stream_workspaces(hipStream_t st);
 
