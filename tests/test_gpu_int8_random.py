@@ -110,3 +110,16 @@ def test_rewritten_operands_and_folded_zero_points(orc, plan, tile, ring, M, K, 
     v = orc.mbqm(want.astype(np.int32), np.broadcast_to(c["mult"], want.shape),
                  -np.broadcast_to(c["shift"], want.shape), orc.HALF_AWAY_FROM_ZERO).astype(np.int64)
     assert np.array_equal(out.cpu().numpy().astype(np.int64), np.clip(v + zp, 0, 255))
+
+
+@pytest.mark.parametrize("M,K,N,zp", [(33, 1024, 64, 0), (65, 1088, 130, 0), (200, 1153, 130, 5), (1000, 1030, 300, 0),
+                                      (1024, 1088, 1024, 0), (1024, 2111, 1024, 9)])
+def test_k_shared_inside_a_workgroup(M, K, N, zp):
+    """64 x 64 tiles with K in two and four runs of unequal length, on either side of 64 and 256 tiles; whole numbers."""
+    import torch
+    g = torch.Generator().manual_seed(M + K + N)
+    a = torch.randint(-128, 128, (M, K), generator=g, dtype=torch.int32).to(torch.int8)
+    b = torch.randint(-128, 128, (N, K), generator=g, dtype=torch.int32).to(torch.int8)
+    out = M_.i8mm_launch(a.cuda(), b.cuda(), None, right_transpose=True, input_zp=zp, right_zp=-zp)
+    want = (a.double() - zp) @ (b.double() + zp).T  # exact: |sum| < 2^53
+    assert np.array_equal(out.cpu().numpy().astype(np.int64), want.numpy().astype(np.int64))

@@ -188,15 +188,18 @@ constexpr int MID_M = 128, MID_N = 128, MID_K = 64;
 // outputs instead of 64
 constexpr int mid_stage_bytes(int bt) { return 2 * bt * MID_K; }  // 16 KiB / 8 KiB
 constexpr int mid_stride(int bt) { return bt / 2 + 4; }  // dwords per row of an epilogue strip (16-byte aligned rows)
-constexpr int mid_lds_bytes(int nst, int bt = 128) {
-  return nst * mid_stage_bytes(bt) > 4 * (bt / 2) * mid_stride(bt) * 4 ? nst * mid_stage_bytes(bt)
-                                                                         : 4 * (bt / 2) * mid_stride(bt) * 4;
+constexpr int mid_lds_bytes(int nst, int bt = 128, int kg = 1) {
+  return kg * (nst * mid_stage_bytes(bt) > 4 * (bt / 2) * mid_stride(bt) * 4 ? nst * mid_stage_bytes(bt)
+                                                                             : 4 * (bt / 2) * mid_stride(bt) * 4);
 }
 
 // MID_NST = stages in the LDS ring: 4 (two workgroups per CU) when there are more tiles than CUs, 8 when every
 // workgroup has a CU to itself -- a short grid is bound by the bytes it keeps in flight.
-template <int MID_NST, int BT, bool ZP>
-__global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m, int tiles_n, int per_xcd) {
+// KG = groups of four waves that share a workgroup's K (1, 2 or 4): each has a ring of its own over its run of stages,
+// and the sums meet in LDS (whole numbers, any order).  For grids that leave CUs idle, where a workgroup's time is its
+// chain of stages (the choice and its figures are where it is launched).
+template <int MID_NST, int BT, bool ZP, int KG = 1>
+__global__ __launch_bounds__(256 * KG) void i8_gemm_mid_kernel(I8Args a, int tiles_m, int tiles_n, int per_xcd) {
   constexpr int WT = BT / 2;                       // a wave's square of outputs: 64 or 32
   constexpr int NB = WT / 32;                      // 32x32 MFMA blocks per side of it
   constexpr int MID_STAGE = mid_stage_bytes(BT);
@@ -208,7 +211,8 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
   constexpr int LPS = 2 * LOADS;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wave_all & 3, kg = wave_all >> 2;  // wave of its group, group
   const int wm = wave >> 1, wn = wave & 1;
   const int bid = blockIdx.x;
   const int L = (bid & 7) * per_xcd + (bid >> 3);  // each XCD gets a contiguous run of the tile order
@@ -235,10 +239,15 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
     ga[i] = a.A + ra * a.K + chunk * 16;
     gb[i] = a.B + rb * a.K + chunk * 16;
   }
-  const int kt_total = (int)(a.K / MID_K);
+  const int kt_all = (int)(a.K / MID_K);
+  const int kt_total = (kt_all + KG - 1) / KG;  // stages per group: every wave passes as many barriers
+  const int kt_begin = kg * kt_total;           // the last groups may have fewer, down to none
+  const int kt_mine = kt_all - kt_begin;
+  uint8_t *ring = lds + kg * (MID_NST * MID_STAGE);
   auto issue = [&](int kt) {
-    const int64_t koff = (int64_t)(kt < kt_total ? kt : kt_total - 1) * MID_K;  // past the end: harmless re-load
-    uint8_t *sa = lds + (kt % MID_NST) * MID_STAGE, *sb = sa + BT * MID_K;
+    const int k = kt_begin + kt;
+    const int64_t koff = (int64_t)(k < kt_all ? k : kt_all - 1) * MID_K;  // past the end: harmless re-load
+    uint8_t *sa = ring + (kt % MID_NST) * MID_STAGE, *sb = sa + BT * MID_K;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       __builtin_amdgcn_global_load_lds((gptr_t)(ga[i] + koff), (lptr_t)(sa + (i * 4 + wave) * 1024), 16, 0, 0);
@@ -297,16 +306,20 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
         dst[e] = src[(n0 + e) < a.N ? (n0 + e) : (a.N - 1)];
     }
   };
-  load16(a.bias, 0, p_bias);
+  auto load_params = [&]() {
+    load16(a.bias, 0, p_bias);
+    if (a.q31_half_away) {
+      load16(a.rq.mult, a.rq.mult_s, p_mult);
+      load16(a.rq.shift, a.rq.shift_s, p_shift);
+      load16(a.rq.zp, a.rq.zp_s, p_zp);
+    }
+  };
+  if constexpr (KG < 4)  // (sixteen waves have 128 registers each, too few to hold these through the loop)
+    load_params();
   int32_t sum_a[NB], sum_b[NB];  // ZP: this lane's half of the sum of row i * 32 + lane % 32 of either operand
 #pragma unroll
   for (int i = 0; i < NB; ++i)
     sum_a[i] = sum_b[i] = 0;
-  if (a.q31_half_away) {
-    load16(a.rq.mult, a.rq.mult_s, p_mult);
-    load16(a.rq.shift, a.rq.shift_s, p_shift);
-    load16(a.rq.zp, a.rq.zp_s, p_zp);
-  }
 #pragma unroll
   for (int s0 = 0; s0 < MID_NST - 1; ++s0)
     issue(s0);
@@ -315,7 +328,9 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
     __builtin_amdgcn_s_waitcnt(waitcnt_vm((MID_NST - 2) * LPS));
     __builtin_amdgcn_s_barrier();  // everyone's share of stage kt is in LDS; everyone is done with stage kt - 1
     issue(kt + MID_NST - 1);
-    const uint8_t *st = lds + (kt % MID_NST) * MID_STAGE;
+    if (KG > 1 && kt >= kt_mine)
+      continue;
+    const uint8_t *st = ring + (kt % MID_NST) * MID_STAGE;
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       i32x4 fa[NB], fb[NB];
@@ -349,7 +364,7 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
   if constexpr (ZP) {
 #pragma unroll
     for (int j = 0; j < NB; ++j) {  // lane l: column l % 32 of block column j, both k halves
-      const int32_t col = a.kzz - a.izp * (sum_b[j] + __shfl_xor(sum_b[j], 32, 64));
+      const int32_t col = (kg == 0 ? a.kzz : 0) - a.izp * (sum_b[j] + __shfl_xor(sum_b[j], 32, 64));
 #pragma unroll
       for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -370,7 +385,7 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
       }
     }
   }
-  int32_t *strip = (int32_t *)lds + wave * (WT * MID_STRIDE);
+  int32_t *strip = (int32_t *)lds + wave_all * (WT * MID_STRIDE);
 #pragma unroll
   for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -378,7 +393,16 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         strip[(i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * MID_STRIDE + j * 32 + (lane & 31)] = acc[i][j][r];
-  // a wave only reads what it wrote: no barrier, the LDS counter orders it
+  if constexpr (KG == 4) {
+    if (kg == 0)
+      load_params();
+  }
+  if constexpr (KG > 1) {
+    __syncthreads();  // the first group reads all strips of its rows
+    if (kg != 0)
+      return;
+  }
+  // KG == 1: a wave only reads what it wrote: no barrier, the LDS counter orders it
   int32_t p_half[16];
   if (a.q31_half_away) {
 #pragma unroll
@@ -395,7 +419,10 @@ __global__ __launch_bounds__(256) void i8_gemm_mid_kernel(I8Args a, int tiles_m,
     int32_t v[16];
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) {
-      const i32x4 t = *(const i32x4 *)(strip + row * MID_STRIDE + cc * 16 + q4 * 4);
+      i32x4 t = *(const i32x4 *)(strip + row * MID_STRIDE + cc * 16 + q4 * 4);
+#pragma unroll
+      for (int g = 1; g < KG; ++g)
+        t += *(const i32x4 *)(strip + (g * 4 * WT + row) * MID_STRIDE + cc * 16 + q4 * 4);
       v[q4 * 4 + 0] = t[0] + p_bias[q4 * 4 + 0];
       v[q4 * 4 + 1] = t[1] + p_bias[q4 * 4 + 1];
       v[q4 * 4 + 2] = t[2] + p_bias[q4 * 4 + 2];
@@ -1158,24 +1185,37 @@ int i8mm_launch(const void *d_a, int a_unsigned, const void *d_b, int b_unsigned
     const int tiles_m = (int)((M + bt - 1) / bt), tiles_n = (int)((N + bt - 1) / bt);
     const int per_xcd = (tiles_m * tiles_n + 7) / 8;
     const dim3 grid((unsigned)(per_xcd * 8));
-#define MI_MID(NST, BT, ZP)                                                                                        \
+    const int64_t tiles = (int64_t)tiles_m * tiles_n;
+    // K in 2 or 4 runs inside a workgroup while there is at most one workgroup a CU (the eight-wave form holds a CU to
+    // itself: 384 tiles of K = 4544 took 5 us longer with it) and a run is worth its join (K = 512: 0.1 to 0.4 us
+    // slower).  Four runs where the fragments also pass through the vector unit (zero points) or few tiles leave the
+    // memory idle.  us with 1 / 2 / 4 runs, signed: 128x4096x1024 11.7 / 10.2 / 9.5, 333x3072x1000 11.2 / 10.4 / 10.9,
+    // 128x4096x4096 12.8 / 11.8 / 12.7; unsigned: 333x3072x1000 15.3 / 13.0 / 11.9, 64x8192x4096 32.0 / 25.7 / 22.2
+    const int kg = tiles > 256 || Kp < 1024 ? 1 : (zp || tiles <= 64) ? 4 : 2;
+#define MI_MID(NST, BT, ZP, KG)                                                                                    \
   {                                                                                                                \
     static LdsLimitOnce lds_limit;                                                                                 \
-    lds_limit.ensure((const void *)i8_gemm_mid_kernel<NST, BT, ZP>, 160 * 1024);                                   \
-    i8_gemm_mid_kernel<NST, BT, ZP><<<grid, dim3(256), mid_lds_bytes(NST, BT), stream>>>(a, tiles_m, tiles_n, per_xcd); \
+    lds_limit.ensure((const void *)i8_gemm_mid_kernel<NST, BT, ZP, KG>, 160 * 1024);                               \
+    i8_gemm_mid_kernel<NST, BT, ZP, KG><<<grid, dim3(256 * KG), mid_lds_bytes(NST, BT, KG), stream>>>(             \
+        a, tiles_m, tiles_n, per_xcd);                                                                             \
   }
-    if (ring == 64 && zp)
-      MI_MID(4, 64, true)
-    else if (ring == 64)
-      MI_MID(4, 64, false)
-    else if (ring == 8 && zp)
-      MI_MID(8, 128, true)
-    else if (ring == 8)
-      MI_MID(8, 128, false)
-    else if (zp)
-      MI_MID(4, 128, true)
-    else
-      MI_MID(4, 128, false)
+#define MI_MID_ZP(NST, BT, KG) \
+  if (zp)                      \
+    MI_MID(NST, BT, true, KG)  \
+  else                         \
+    MI_MID(NST, BT, false, KG)
+    if (ring == 64 && kg == 4) {
+      MI_MID_ZP(4, 64, 4)
+    } else if (ring == 64 && kg == 2) {
+      MI_MID_ZP(4, 64, 2)
+    } else if (ring == 64) {
+      MI_MID_ZP(4, 64, 1)
+    } else if (ring == 8) {
+      MI_MID_ZP(8, 128, 1)
+    } else {
+      MI_MID_ZP(4, 128, 1)
+    }
+#undef MI_MID_ZP
 #undef MI_MID
   }
   MI_HIP(hipGetLastError());
