@@ -281,6 +281,7 @@ int cast_launch(const mi_cast_attr *c, const void *d_in, void *d_out, int64_t n,
     cast_kernel<IN, OUT><<<grid, dim3(256), 0, stream>>>(a);      \
   else
   // the conversions on either side of the matmuls
+  MI_CAST(MI_ST_F32, MI_ST_F32)
   MI_CAST(MI_ST_F32, MI_ST_BF16)
   MI_CAST(MI_ST_BF16, MI_ST_F32)
   MI_CAST(MI_ST_F32, MI_ST_F16)
