@@ -123,3 +123,65 @@ def test_k_shared_inside_a_workgroup(M, K, N, zp):
     out = M_.i8mm_launch(a.cuda(), b.cuda(), None, right_transpose=True, input_zp=zp, right_zp=-zp)
     want = (a.double() - zp) @ (b.double() + zp).T  # exact: |sum| < 2^53
     assert np.array_equal(out.cpu().numpy().astype(np.int64), want.numpy().astype(np.int64))
+
+
+def _kn_products(n):
+    """n [K, N] products with a K that has to be padded: operands, their rewriting goes through the stream's scratch."""
+    import torch
+    g = torch.Generator().manual_seed(n)
+    sets = []
+    for i in range(n):
+        a = torch.randint(-128, 128, (70 + i, 1000), generator=g, dtype=torch.int32).to(torch.int8)
+        b = torch.randint(-128, 128, (1000, 300), generator=g, dtype=torch.int32).to(torch.int8)
+        sets.append((a.cuda(), b.cuda(), (a.double() @ b.double()).to(torch.int32)))
+    return sets
+
+
+def test_threads_on_one_stream_keep_their_rewritten_operands():
+    """Several threads launch on the same stream: the rewriting and the product of one call stay together."""
+    import threading
+    import torch
+    stream = torch.cuda.Stream()
+    sets = _kn_products(4)
+    torch.cuda.synchronize()
+    outs = [None] * len(sets)
+
+    def work(i):
+        with torch.cuda.stream(stream):
+            outs[i] = [M_.i8mm_launch(sets[i][0], sets[i][1]) for _ in range(40)]
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(sets))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for (_, _, want), got in zip(sets, outs):
+        assert len(got) == 40
+        for y in got:
+            assert torch.equal(y.cpu(), want)
+
+
+def test_captured_product_has_scratch_of_its_own():
+    """A graph replayed on another stream runs beside eager calls on the stream that it was captured on."""
+    import torch
+    (a, b, want), (a2, b2, want2) = _kn_products(2)
+    cap, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(cap):
+        M_.i8mm_launch(a, b)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=cap):
+        y = M_.i8mm_launch(a, b)
+    for _ in range(5):
+        y.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            graph.replay()
+        with torch.cuda.stream(cap):
+            eager = [M_.i8mm_launch(a2, b2) for _ in range(8)]
+        torch.cuda.synchronize()
+        assert torch.equal(y.cpu(), want)
+        for e in eager:
+            assert torch.equal(e.cpu(), want2)

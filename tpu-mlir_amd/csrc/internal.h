@@ -4,6 +4,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <string>
 
 #include "../../include/tpumlir_amd.h"
@@ -172,7 +173,7 @@ int a16_launch_group(const mi_a16_weight *const *ws, int n, const uint16_t *d_x,
 
 // library-owned scratch, one buffer per (device, stream, purpose) (workspace.hip); contents are whatever the last
 // user left
-enum { WS_SPLIT_K = 0, WS_DYNAMIC_QUANT = 1, WS_F8_OPERANDS = 2, WS_ROWS32_SPLIT = 3, WS_I8_OPERANDS = 4 };
+enum { WS_SPLIT_K = 0, WS_DYNAMIC_QUANT = 1, WS_F8_OPERANDS = 2, WS_ROWS32_SPLIT = 3, WS_I8_OPERANDS = 4, WS_COUNT };
 // WS_ROWS32_SPLIT, shared by the few-row kernels that split K over workgroups (A16 and INT8): arrival counters, then
 // one 32 x 32 block of partial sums per workgroup.  Always asked for at this one size, so it is never re-allocated.
 constexpr int R32_SPLIT_MAX_WGS = 256;          // workgroups of a split launch, at most
@@ -181,18 +182,27 @@ constexpr int R32_SPLIT_COUNTER_BYTES = 1024;   // one counter per block of a sp
 // for the same size)
 int stream_workspace(hipStream_t st, int purpose, size_t bytes, void **out, bool zero_fresh = false);
 long workspace_allocations();
-// Scratch of one launch that a stream under capture may also need, and whose size follows the caller's operands: up to
-// 64 MiB of the stream's buffer (sizes in powers of two, so that what growing retires stays below what is in use), and
-// beyond that, or where the buffer would have to grow under capture, memory of this launch alone from the runtime's
-// stream-ordered pool.  (That pool for every call, as it was: it gives its memory back at each synchronization and takes
-// about 60 us to get it again.)
+// Scratch of one call that enqueues a producer and a consumer of it, and whose size follows the caller's operands: up
+// to 64 MiB of the stream's buffer (sizes in powers of two, so that what growing retires stays below what is in use).
+// The two launches must not be interleaved with those of another thread on the same stream, so a lock is held from
+// get() to release().  Memory of the call alone, from the runtime's stream-ordered pool, is taken beyond that size,
+// under capture of a stream that is not declared below (its graph may be replayed on another stream, beside this
+// stream's own calls) and on the per-thread stream (one handle, many streams).  (That pool for every call, as it was: it gives its memory back at each
+// synchronization and takes about 60 us to get it again.)
 struct ScratchBytes {
   void *ptr = nullptr;
   bool own = false;
   hipStream_t stream = nullptr;
+  std::unique_lock<std::mutex> use;
   int get(hipStream_t st, int purpose, size_t bytes);
   int release();  // after the last launch that uses it
+  ~ScratchBytes() {
+    if (own)
+      (void)hipFreeAsync(ptr, stream);
+  }
 };
+// for owners of private streams: graphs captured on it are only replayed on it, until release_stream_workspaces()
+void stream_replays_in_order(hipStream_t st);
 // 8-bit matmul operands in the layout of the tile kernels, both in one launch (operand_copy.hip); src null: none
 struct OperandCopy {
   const uint8_t *src;

@@ -294,6 +294,7 @@ int mi_module_create(mi_module **out) {
   MI_REQUIRE(mi_device_count() > 0, MI_HIP_ERROR, "mi_module_create: no GPU visible");
   std::unique_ptr<mi_module> m(new mi_module());
   MI_HIP(hipStreamCreate(&m->stream));
+  mi::stream_replays_in_order(m->stream);  // invoke() replays where it captured
   *out = m.release();
   return MI_SUCCESS;
 }

@@ -9,6 +9,7 @@
 // stream is being captured into a graph: run a shape once eagerly before capturing it.
 #include <map>
 #include <mutex>
+#include <set>
 #include <tuple>
 #include <vector>
 
@@ -58,31 +59,47 @@ int stream_workspace(hipStream_t st, int purpose, size_t bytes, void **out, bool
   return MI_SUCCESS;
 }
 
+namespace {
+std::mutex g_scratch_use[WS_COUNT];  // taken before g_mutex, never after it
+std::set<hipStream_t> g_replay_in_order;
+}  // namespace
+
+void stream_replays_in_order(hipStream_t st) {
+  std::lock_guard<std::mutex> lock(g_mutex);
+  g_replay_in_order.insert(st);
+}
+
 int ScratchBytes::get(hipStream_t st, int purpose, size_t bytes) {
   stream = st;
   size_t want = 1 << 16;
   while (want < bytes)
     want *= 2;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  bool kept = want <= ((size_t)64 << 20);
-  if (kept && hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {
+  const bool capturing = hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+  bool kept = st != hipStreamPerThread && want <= ((size_t)64 << 20);
+  if (kept && capturing) {
     int dev = 0;
     MI_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lock(g_mutex);
     const auto it = g_bufs.find(std::make_tuple(dev, st, purpose));
-    kept = it != g_bufs.end() && it->second.bytes >= want;
+    kept = g_replay_in_order.count(st) && it != g_bufs.end() && it->second.bytes >= want;
   }
-  if (kept)
+  if (kept) {
+    use = std::unique_lock<std::mutex>(g_scratch_use[purpose]);
     return stream_workspace(st, purpose, want, &ptr);
+  }
   MI_HIP(hipMallocAsync(&ptr, bytes, st));
   own = true;
   return MI_SUCCESS;
 }
 
 int ScratchBytes::release() {
-  if (own)
+  if (use.owns_lock())
+    use.unlock();
+  if (own) {
+    own = false;
     MI_HIP(hipFreeAsync(ptr, stream));
-  own = false;
+  }
   return MI_SUCCESS;
 }
 
@@ -96,6 +113,7 @@ void release_stream_workspaces(hipStream_t st) {
   if (hipGetDevice(&dev) != hipSuccess)
     return;
   std::lock_guard<std::mutex> lock(g_mutex);
+  g_replay_in_order.erase(st);
   for (auto it = g_bufs.begin(); it != g_bufs.end();) {
     if (std::get<0>(it->first) == dev && std::get<1>(it->first) == st) {
       (void)hipStreamSynchronize(st);
