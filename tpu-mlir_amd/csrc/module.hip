@@ -36,21 +36,9 @@ struct DevMem {
   DevMem &operator=(const DevMem &) = delete;
 };
 
-// pinned host memory that kernels read and write over the bus; only grows
+// pinned host memory that kernels read and write over the bus
 struct HostMem {
-  void *ptr = nullptr;
-  size_t cap = 0;
-  int reserve(size_t bytes) {
-    if (bytes <= cap)
-      return MI_SUCCESS;
-    if (ptr)
-      (void)hipHostFree(ptr);
-    ptr = nullptr;
-    cap = 0;
-    MI_HIP(hipHostMalloc(&ptr, bytes, hipHostMallocDefault));
-    cap = bytes;
-    return MI_SUCCESS;
-  }
+  float *ptr = nullptr;
   ~HostMem() {
     if (ptr)
       (void)hipHostFree(ptr);
@@ -59,6 +47,13 @@ struct HostMem {
   HostMem(const HostMem &) = delete;
   HostMem &operator=(const HostMem &) = delete;
 };
+
+// Tensors of up to this many elements cross the bus inside the conversion kernel, which reads or writes the floats in
+// pinned host memory: one launch where a copy command to or from pageable memory, a launch and the gap between them
+// were.  Larger ones are copied by the runtime, whose copies overlap with its own staging.  A decoder block for one
+// token (4096 in, outputs of 2 x 4096, 11008 and 4096 read back): 169 -> 119 us.  The two buffers are allocated with
+// the module, beside its weights, and not in its first pass, which grew by 70 us when they were.
+constexpr int64_t SMALL_TENSOR_ELEMS = 1 << 16;
 
 struct Tensor {
   std::string name;
@@ -114,13 +109,13 @@ struct mi_module {
   bool graph_tried = false;
   DevMem staging;  // float staging for set_tensor / get_tensor of large tensors
   size_t staging_bytes = 0;
-  HostMem host_in, host_out;  // the same for small ones
-  bool host_in_busy = false;  // a conversion that reads host_in may still be on its way
+  HostMem host;               // the same for small ones: floats on their way in, then floats on their way out
+  bool host_in_busy = false;  // a conversion that reads them may still be on its way
   std::unique_ptr<DevMem> arena;  // one allocation shared by the activations whose lifetimes do not overlap
   mi_module_hook before = nullptr, after = nullptr;
   void *hook_user = nullptr;
   ~mi_module() {
-    if (host_in_busy)  // host_in is freed below
+    if (host_in_busy)  // the memory is freed below
       (void)hipStreamSynchronize(stream);
     if (exec)
       (void)hipGraphExecDestroy(exec);
@@ -294,6 +289,7 @@ int mi_module_create(mi_module **out) {
   MI_REQUIRE(mi_device_count() > 0, MI_HIP_ERROR, "mi_module_create: no GPU visible");
   std::unique_ptr<mi_module> m(new mi_module());
   MI_HIP(hipStreamCreate(&m->stream));
+  MI_HIP(hipHostMalloc((void **)&m->host.ptr, 2 * SMALL_TENSOR_ELEMS * sizeof(float), hipHostMallocDefault));
   mi::stream_replays_in_order(m->stream);  // invoke() replays where it captured
   *out = m.release();
   return MI_SUCCESS;
@@ -551,12 +547,6 @@ int mi_module_add_cast(mi_module *m, const char *input, const char *output, cons
   return MI_SUCCESS;
 }
 
-// Tensors of up to this many elements cross the bus inside the conversion kernel, which reads or writes the floats in
-// pinned host memory: one launch where a copy command to or from pageable memory, a launch and the gap between them
-// were.  Larger ones are copied by the runtime, whose copies overlap with its own staging.  A decoder block for one
-// token (4096 in, outputs of 2 x 4096, 11008 and 4096 read back): 169 -> 119 us.
-constexpr int64_t SMALL_TENSOR_ELEMS = 1 << 16;
-
 int mi_module_set_tensor(mi_module *m, const char *name, const float *data, int64_t num_elem) {
   int idx, rc;
   if ((rc = find(m, name, &idx)))
@@ -568,12 +558,10 @@ int mi_module_set_tensor(mi_module *m, const char *name, const float *data, int6
       MI_HIP(hipStreamSynchronize(m->stream));
       m->host_in_busy = false;
     }
-    if ((rc = m->host_in.reserve((size_t)t.n * 4)))
-      return rc;
-    memcpy(m->host_in.ptr, data, (size_t)t.n * 4);
+    memcpy(m->host.ptr, data, (size_t)t.n * 4);
     mi_cast_attr c = plain_cast(MI_ST_F32, t.st, t.n);
     // whatever uses the tensor next is ordered behind this on the module's stream
-    if ((rc = cast_launch(&c, m->host_in.ptr, t.ptr(), t.n, 1.0f, 1.0f, false, m->stream)))
+    if ((rc = cast_launch(&c, m->host.ptr, t.ptr(), t.n, 1.0f, 1.0f, false, m->stream)))
       return rc;
     m->host_in_busy = true;
     return MI_SUCCESS;
@@ -660,14 +648,12 @@ static int get_tensor_impl(mi_module *m, const char *name, float *out, int64_t n
              "as an output before planning to keep it");
   const void *src = t.ptr();
   if (t.n <= SMALL_TENSOR_ELEMS) {
-    if ((rc = m->host_out.reserve((size_t)t.n * 4)))
-      return rc;
     mi_cast_attr c = plain_cast(t.st, MI_ST_F32, t.n);
-    if ((rc = cast_launch(&c, src, m->host_out.ptr, t.n, 1.0f, 1.0f, false, m->stream)))
+    if ((rc = cast_launch(&c, src, m->host.ptr + SMALL_TENSOR_ELEMS, t.n, 1.0f, 1.0f, false, m->stream)))
       return rc;
     MI_HIP(hipStreamSynchronize(m->stream));
     m->host_in_busy = false;
-    memcpy(out, m->host_out.ptr, (size_t)t.n * 4);
+    memcpy(out, m->host.ptr + SMALL_TENSOR_ELEMS, (size_t)t.n * 4);
     scale_quantized(t, scaled, out);
     return MI_SUCCESS;
   }
