@@ -99,8 +99,8 @@ def test_tflite_lshift_with_left_shifts(orc, rmode):
     want = _sat(orc.mbqm(x, np.broadcast_to(mult, x.shape), np.broadcast_to(-sh, x.shape), rmode).astype(np.int64)
                 + zp[None, :], -128, 127)
     assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
-    # fused: INT8 matmul whose accumulators take the same per-channel parameters (mid-size tiled kernel and, through
-    # K % 64 != 0, the register-staged one)
+    # fused: INT8 matmul whose accumulators take the same per-channel parameters (mid-size tiled kernel, as it
+    # stands and, through K % 64 != 0, behind the operand rewrite)
     for M, K in ((130, 256), (33, 200)):
         c = S.int8_matmul(M, K, C_, seed=K)
         acc = torch.empty((M, C_), dtype=torch.int32, device="cuda")

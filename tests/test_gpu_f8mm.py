@@ -125,7 +125,7 @@ def test_f8_matmul_saturation_ties_and_step_narrowing(orc):
                            np.array([1e4, 3e38, 149.3, 154.6, 154.7, 1e-6, 0.0], np.float32)])
     cand = np.concatenate([cand, -cand]).astype(np.float32)
     N = cand.size
-    for K in (64, 48):                                      # the ring kernel and the register-staged one
+    for K in (64, 48):                                      # the ring kernel as it stands and behind the operand rewrite
         a = np.zeros((3, K), np.uint8)
         b = np.zeros((K, N), np.uint8)
         af, bf = orc.f8e4m3_to_f32(a), orc.f8e4m3_to_f32(b)

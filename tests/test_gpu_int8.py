@@ -108,7 +108,7 @@ def test_zero_points_unsigned_operands_relu_and_int16(orc):
 @pytest.mark.parametrize("rt", [True, False])
 def test_large_tile_path_unsigned_zero_points_relu_ragged_edges(orc, plan, rt, tile):
     """Each of the GEMM kernels (256x256 direct-to-LDS tiles; 128x128 tiles with a ring of 8 or 4 stages and the
-    64x64-tile form of the same kernel; register-staged 128x128) on a shape all of them accept (M, N >= 128,
+    64x64-tile form of the same kernel; -1: the size rule's own choice among them) on a shape all of them accept (M, N >= 128,
     K % 128 == 0), with everything the small cases cover: unsigned operands, both zero points, bias, relu with a
     limit, a ragged last tile in M and N, per-channel Q31 requant with per-channel output zero points, and the int32
     side output."""
