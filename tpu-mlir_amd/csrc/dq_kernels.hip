@@ -198,6 +198,102 @@ __global__ __launch_bounds__(256) void dq_act_kernel(DqActJob ja, DqActJob jb, i
   }
 }
 
+// The same for few rows, where the kernel above leaves most of the chip idle and its time is the chain of conversions of
+// one thread (16 of them for groups of 128; an E4M3 or E2M1 conversion is some 50 instructions): a piece of eight
+// elements goes to four threads, which all look for the largest and convert two each, the pair that is adjacent in the
+// stored order.  A workgroup takes eight rows of a unit.  Not for [K][rows] operands.
+template <int DT, int BITS, int FLAV>
+__global__ __launch_bounds__(256) void dq_act_few_kernel(DqActJob j, int g, int G, float imax) {
+  using H = Half16<DT>;
+  const int p = threadIdx.x & 3, l8 = (threadIdx.x >> 2) & 7, row = (int)(blockIdx.x & 1) * 8 + (threadIdx.x >> 5);
+  const int64_t u = blockIdx.x >> 1;  // two workgroups a unit: below j.units
+  const int steps = g >= 64 ? g / 64 : 1;
+  const int64_t per_block = g >= 64 ? G : j.K / 64;
+  const int64_t mb = u / per_block;
+  const int c0 = (int)(u - mb * per_block) * steps;
+  const int64_t m = mb * 16 + row;
+  const bool live = m < j.rows;
+  auto load8 = [&](int step) {
+    u32x4 v = {0, 0, 0, 0};
+    if (live)
+      __builtin_memcpy(&v, j.x + m * j.K + (int64_t)(c0 + step) * 64 + l8 * 8, 16);
+    return v;
+  };
+  float amax = (float)1e-8;
+  auto take_max = [&](const u32x4 &v) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const float f = fabsf(H::to_f32((uint16_t)v[d])), h = fabsf(H::to_f32((uint16_t)(v[d] >> 16)));
+      amax = amax > f ? amax : f;
+      amax = amax > h ? amax : h;
+    }
+  };
+  constexpr int HELD = 2;
+  u32x4 held[HELD];
+#pragma unroll
+  for (int s = 0; s < HELD; ++s)
+    if (s < steps) {
+      held[s] = load8(s);
+      take_max(held[s]);
+    }
+  for (int s = HELD; s < steps; ++s)
+    take_max(load8(s));
+  const int span = g == 32 ? 16 : 32;  // lanes of a row's group
+  for (int o = span >> 1; o >= 4; o >>= 1) {
+    const float other = __shfl_xor(amax, o, 64);
+    amax = amax > other ? amax : other;
+  }
+  const float step_size = amax / imax;
+  int sum = 0;
+  float fsum = 0.0f;
+  auto convert = [&](uint32_t bits) {
+    const float f = H::to_f32((uint16_t)bits);
+    int code;
+    if constexpr (FLAV == FLAV_INT) {
+      code = (int)roundf(f / amax * imax);
+      sum += code;
+    } else {
+      if constexpr (FLAV == FLAV_F8)
+        code = (int)f8e4m3_from_f32(__fdiv_rn(f, step_size));
+      else
+        code = (int)f4_code_as_f8(f4e2m1_from_f32(__fdiv_rn(f, step_size)));
+      fsum += f8e4m3_to_f32((uint32_t)code);
+    }
+    return (uint32_t)(code & 0xff);
+  };
+  auto emit = [&](int step, const u32x4 &v) {
+    uint32_t first, second;
+    if constexpr (BITS == 4) {  // elements p and p + 4: dq_slot puts them at 2 p and 2 p + 1
+      const uint32_t a = p < 2 ? v[0] : v[1], b = p < 2 ? v[2] : v[3];
+      first = (p & 1) ? a >> 16 : a;
+      second = (p & 1) ? b >> 16 : b;
+    } else {
+      const uint32_t a = p < 2 ? (p == 0 ? v[0] : v[1]) : (p == 2 ? v[2] : v[3]);
+      first = a;
+      second = a >> 16;
+    }
+    const uint32_t lo = convert(first), hi = convert(second);
+    uint8_t *dst = j.aq + (mb * (j.K / 64) + c0 + step) * 1024 + ((l8 & 3) * 16 + row) * 16 + (l8 >> 2) * 8 + 2 * p;
+    *(uint16_t *)dst = (uint16_t)(live ? lo | (hi << 8) : 0u);
+  };
+#pragma unroll
+  for (int s = 0; s < HELD; ++s)
+    if (s < steps)
+      emit(s, held[s]);
+  for (int s = HELD; s < steps; ++s)
+    emit(s, load8(s));
+  for (int o = span >> 1; o > 0; o >>= 1) {
+    sum += __shfl_xor(sum, o, 64);
+    fsum += __shfl_xor(fsum, o, 64);
+  }
+  if ((threadIdx.x & (span - 1)) == 0) {
+    const int64_t gi = g >= 64 ? u - mb * per_block : (int64_t)c0 * 2 + (l8 >> 2);
+    const int64_t at = (mb * G + gi) * 16 + row;
+    j.as_t[at] = live ? step_size : 0.0f;
+    j.asum_t[at] = !live ? 0 : FLAV == FLAV_INT ? sum : __float_as_int(fsum);
+  }
+}
+
 struct DqArgs {
   const u32x4 *qw;
   const uint32_t *sz_t;      // 4-bit
@@ -965,6 +1061,7 @@ int a16_dq_launch(const mi_a16_weight *w, int dq_type, const uint16_t *d_x, int6
   const DqActJob job = {d_x, aq, as_t, asum_t, M, w->K, m_blocks * (g >= 64 ? G : w->K / 64), 0};
   const DqActJob none = {};
   const dim3 act_grid((unsigned)((job.units + 1) / 2));
+  const bool few_units = job.units <= 768;
   const bool tiled = dq_takes_tiles(m_blocks, w->row_blocks, w->K);
   const bool f16 = w->dtype == MI_DT_F16;
   DqArgs a;
@@ -992,7 +1089,10 @@ int a16_dq_launch(const mi_a16_weight *w, int dq_type, const uint16_t *d_x, int6
   const int gemm_waves = (wo == DQ_WAVES || wo == 2 * DQ_WAVES) ? wo : ((int64_t)w->row_blocks * m_blocks <= 256 ? 2 * DQ_WAVES : DQ_WAVES);
 #define MI_DQ_RUN(DT_, BITS_, FLAV_)                                                                             \
   {                                                                                                             \
-    dq_act_kernel<DT_, BITS_, FLAV_><<<act_grid, dim3(256), 0, stream>>>(job, none, g, G, imax);                \
+    if (few_units)                                                                                              \
+      dq_act_few_kernel<DT_, BITS_, FLAV_><<<dim3((unsigned)(2 * job.units)), dim3(256), 0, stream>>>(job, g, G, imax); \
+    else                                                                                                        \
+      dq_act_kernel<DT_, BITS_, FLAV_><<<act_grid, dim3(256), 0, stream>>>(job, none, g, G, imax);              \
     if (!tiled) {                                                                                               \
       static LdsLimitOnce lds_limit;                                                                            \
       lds_limit.ensure((const void *)dq_gemm_kernel<DT_, BITS_, FLAV_>, 160 * 1024);                            \
