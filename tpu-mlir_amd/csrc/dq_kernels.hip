@@ -1061,6 +1061,8 @@ int a16_dq_launch(const mi_a16_weight *w, int dq_type, const uint16_t *d_x, int6
   const DqActJob job = {d_x, aq, as_t, asum_t, M, w->K, m_blocks * (g >= 64 ? G : w->K / 64), 0};
   const DqActJob none = {};
   const dim3 act_grid((unsigned)((job.units + 1) / 2));
+  // dq_act_kernel / dq_act_few_kernel, both with the product, us by units: 256 INT 10.2 / 10.4, F4 13.0 / 10.9; 512 INT
+  // 12.6 / 12.4, F4 15.9 / 14.7; 1024 INT 20.3 / 20.6, groups of 64 23.7 / 24.7, F4 26.1 / 25.9; 2048 F4 30.7 / 32.5
   const bool few_units = job.units <= 768;
   const bool tiled = dq_takes_tiles(m_blocks, w->row_blocks, w->K);
   const bool f16 = w->dtype == MI_DT_F16;
