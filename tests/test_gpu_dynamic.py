@@ -521,6 +521,13 @@ def test_dynamic_tiles(orc, plan, bits, M, K, N, g, bias, dq):
         assert np.array_equal(out, orc.f32_to_bf16(want))
 
 
+@pytest.mark.parametrize("bits,M,K,N,g,dq", [(4, 512, 1536, 16, 32, "INT"), (4, 513, 1536, 16, 32, "INT"), (4, 1024, 1536, 16, 128, "F4"),
+                                             (4, 1025, 1536, 16, 128, "F4"), (8, 505, 1536, 16, 64, "INT"), (8, 520, 1536, 16, 64, "F8")])
+def test_dynamic_quantizers_at_their_line(orc, plan, bits, M, K, N, g, dq):
+    """768 units of 16 rows by a group (or chunk), the few-row quantizer's last, and just past them."""
+    test_dynamic_tiles(orc, plan, bits, M, K, N, g, False, dq)
+
+
 def _f8_weights(cfg):
     """Dequantized E4M3 weights (|values| only matter here), scales per group applied."""
     import torch
